@@ -216,7 +216,9 @@ int plan_contraction_impl( int64_t            num_loops,
                            int32_t            ktype_last_touch,
                            bool               allow_split,
                            ContractionPlan  & plan,
-                           DevicePlacement  * place ) {
+                           DevicePlacement  * place,
+                           bool               dry = false ) {
+  // dry: tile, load modes and split only, no device memory
   plan = ContractionPlan();
   plan.placed = ( place != nullptr );
 
@@ -757,6 +759,14 @@ int plan_contraction_impl( int64_t            num_loops,
       }
       int64_t const l_ws_bytes = 4 * l_sf * l_span;
       if( l_sf >= 2 && l_size_k / l_sf >= 128 && l_ws_bytes <= ( int64_t( 1 ) << 29 ) ) {
+        if( dry ) {
+          plan.split = (int32_t) l_sf;
+          plan.C = l_size_c;
+          plan.M = l_kern_m;
+          plan.N = l_kern_n;
+          plan.K = l_size_k;
+          return ETIR_SUCCESS;
+        }
         // loop arrays of the partial contraction
         std::vector< int32_t > l_pt;
         std::vector< int64_t > l_psz, l_pl, l_pr, l_pa, l_po;
@@ -834,6 +844,8 @@ int plan_contraction_impl( int64_t            num_loops,
   plan.M = l_kern_m;
   plan.N = l_kern_n;
   plan.K = l_size_k;
+  plan.args.k_affine = l_k_affine ? 1 : 0;
+  if( dry ) return ETIR_SUCCESS;
   // complex: four real products per complex multiply-add
   plan.flops = ( l_cpx ? 8 : 2 ) * l_size_c * l_size_m * l_size_n * l_size_k;
   int64_t const l_esz_out = ( dtype_out == ETIR_BF16 ) ? 2 : ( dtype_out == ETIR_FP64 ? 8 : 4 );
@@ -1062,6 +1074,266 @@ int plan_contraction_impl( int64_t            num_loops,
   return ETIR_SUCCESS;
 }
 
+// Rate (TFLOP/s) a plan's kernel reaches on a full chip, by its tile and its
+// operands' load modes (one or both gathered element by element), measured at
+// 511 to 4095 a side.  `far`: a gathered operand above an XCD's 4 MB L2 whose
+// neighbouring elements are neither along K nor along its rows (measured at
+// 1152 to 8064 a side).  Only for comparing a plan with its packed forms.
+double plan_rate( ContractionPlan const & plan, bool far ) {
+  int const l_s = ( plan.mode_a == LOAD_SCALAR ? 1 : 0 ) + ( plan.mode_b == LOAD_SCALAR ? 1 : 0 );
+  auto by_mode = [&]( double vec, double one, double two, double far_one ) {
+    return l_s == 0 ? vec : ( far ? far_one : ( l_s == 1 ? one : two ) );
+  };
+  switch( plan.tile ) {
+    case TILE_F32_DMA_128x128:  return 135.0;
+    case TILE_F32_128x128:      return by_mode( 112.0, 75.0, 75.0, 16.0 );
+    case TILE_F32_64x64:        return by_mode( 65.0, 30.0, 25.0, 25.0 );
+    case TILE_BF16_DMA_256x256: return plan.mode_a == LOAD_VEC_MN && plan.mode_b == LOAD_VEC_MN ? 1100.0 : 800.0;
+    case TILE_BF16_256x128:     return by_mode( 550.0, 100.0, 95.0, 20.0 );
+    case TILE_BF16_128x128:     return by_mode( 550.0, 50.0, 45.0, 20.0 );
+    case TILE_BF16_64x64:       return by_mode( 300.0, 46.0, 45.0, 25.0 );
+    case TILE_F64_64x64:        return by_mode( 50.0, 48.0, 48.0, 18.0 );
+    default:                    return 0.0;   // not a tile that packing is weighed against
+  }
+}
+
+// estimated time (us): flops at plan_rate over the useful part of the tile
+// grid, or the tensors' bytes at 3.5 TB/s where that is longer
+double plan_us( ContractionPlan const & plan, bool far, double flops, double bytes ) {
+  int64_t l_bm, l_bn;
+  tile_shape( plan.tile, l_bm, l_bn );
+  double const l_tm = double( ( plan.M + l_bm - 1 ) / l_bm ), l_tn = double( ( plan.N + l_bn - 1 ) / l_bn );
+  double const l_tiles = l_tm * l_tn * double( plan.C ) * double( plan.split );
+  double const l_util = double( plan.M ) * double( plan.N ) / ( l_tm * double( l_bm ) * l_tn * double( l_bn ) )
+                      * std::min( 1.0, l_tiles / 256.0 );
+  return std::max( flops / ( plan_rate( plan, far ) * l_util * 1e6 ), bytes / 3.5e6 ) + 5.0;
+}
+
+// Weighs copying one or both operands K-contiguous into a workspace
+// (O((M + N) K) bytes) against reading them in place (O(M N K) loads), and
+// builds the packed contraction where it is clearly faster.
+//
+// In place, an operand without 16-byte runs along its rows or along the K
+// order of the other one is gathered element by element; a K-contiguous copy
+// (rows padded with zeros to whole 16-byte vectors when both are copied) takes
+// the vector tiles and the direct-to-LDS kernels.  A K of several loops that
+// are not adjacent in an operand (table K: 112 against 135 TFLOP/s in fp32)
+// is packed too where the longer kernel pays for the copy.  Measured, in
+// place against packed, copies included:
+//   aecf,bfde->abcd 96,96,84,84,84,84 fp32 (left contiguous along f, right
+//     along e)                               62.3 -> 7.38 ms (14.7 -> 124 TFLOP/s)
+//   the same, 48,48,42,42,42,42 fp64          795 -> 324 us
+//   acd,dbc->ab 384,376,376,384 fp32         1949 -> 466 us
+//   mk,nk->mn, 767 / 1023 / 2047 a side       fp32 61 -> 31, 80 -> 44, 371 -> 160 us
+//                                             bf16 44 -> 23, 58 -> 25, 370 -> 59 us
+// and packed where the rule keeps them in place (a copy costs about 7 us
+// beside its bytes): aecf,bfde->abcd 24,24,12,12,12,12 fp32 12.5 -> 14.0 us,
+// eafd,fbec->abcd 42,42,21,21,21,21 fp32 46 -> 53 us.
+//
+// Never fails: without a gain, or without the memory, the plan stays as it is.
+void try_pack( int64_t            num_loops,
+               int32_t const    * dim_types,
+               int64_t const    * sizes,
+               int64_t const    * strides_left,
+               int64_t const    * strides_right,
+               int64_t const    * strides_out_aux,
+               int64_t const    * strides_out,
+               int32_t            dtype_left,
+               int32_t            dtype_right,
+               int32_t            dtype_comp,
+               int32_t            dtype_out,
+               int32_t            ktype_first_touch,
+               int32_t            ktype_main,
+               int32_t            ktype_last_touch,
+               bool               allow_split,
+               ContractionPlan  & plan ) {
+  if( ktype_main != ETIR_KTYPE_MADD || std::getenv( "ETIR_TILE" ) != nullptr ) return;
+  if( plan.C <= 0 || plan.M <= 0 || plan.N <= 0 || plan.K <= 1 || plan_rate( plan, false ) == 0.0 ) return;
+  auto in_vec = [&]( int32_t m ) { return m == LOAD_VEC_MN || m == LOAD_VEC_K; };
+  bool const l_affine = ( plan.partial ? plan.partial->args.k_affine : plan.args.k_affine ) != 0;
+  if( in_vec( plan.mode_a ) && in_vec( plan.mode_b ) && ( l_affine || dtype_left == ETIR_FP64 ) ) return;
+
+  int64_t const   l_esz  = dtype_bytes( dtype_left );
+  int64_t const   l_vk   = 16 / l_esz;
+  int64_t const * l_st[2] = { strides_left, strides_right };
+
+  // loops an operand runs over (size-1 loops and broadcast ones do not move it)
+  struct Dim { int64_t size, s, id; };
+  std::vector< Dim > l_rows[2], l_k[2];     // C and row loops; K loops: by the operand's stride, outer first
+  double l_bytes[2];
+  for( int l_op = 0; l_op < 2; l_op++ ) {
+    int64_t l_n = 1;
+    for( int64_t l_lo = 0; l_lo < num_loops; l_lo++ ) {
+      if( sizes[l_lo] <= 1 || dim_types[l_lo] == ETIR_DIM_I || dim_types[l_lo] == ETIR_DIM_J ) continue;
+      bool const l_is_k = dim_types[l_lo] == ETIR_DIM_K;
+      if( l_st[l_op][l_lo] == 0 ) {
+        if( l_is_k ) return;                // a K loop that an operand does not move along
+        continue;
+      }
+      ( l_is_k ? l_k : l_rows )[l_op].push_back( { sizes[l_lo], l_st[l_op][l_lo], l_lo } );
+      l_n *= sizes[l_lo];
+    }
+    for( auto * l_set : { &l_rows[l_op], &l_k[l_op] } ) {
+      std::stable_sort( l_set->begin(), l_set->end(), []( Dim const & x, Dim const & y ) { return x.s > y.s; } );
+    }
+    l_bytes[l_op] = double( l_n ) * double( l_esz );
+  }
+
+  double const l_flops = 2.0 * double( plan.C ) * double( plan.M ) * double( plan.N ) * double( plan.K );
+  double const l_out   = double( dtype_bytes( dtype_out ) ) * double( plan.C ) * double( plan.M ) * double( plan.N );
+  // a gathered operand whose unit-stride loop is neither the innermost K loop
+  // of the plan's K order nor the innermost row loop
+  bool l_far = false;
+  for( int l_op = 0; l_op < 2; l_op++ ) {
+    bool const l_is_a = ( l_op == 0 ) != plan.swapped;
+    if( ( l_is_a ? plan.mode_a : plan.mode_b ) != LOAD_SCALAR ) continue;
+    // the K order is that of the kernel's A operand when a K loop is its
+    // unit-stride one, else that of B when one is B's
+    auto unit_k = [&]( int op ) { return !l_k[op].empty() && l_k[op].back().s == 1; };
+    int const l_opa = plan.swapped ? 1 : 0;
+    int const l_order = unit_k( l_opa ) ? l_opa : ( unit_k( 1 - l_opa ) ? 1 - l_opa : l_opa );
+    int64_t const l_kin = l_k[l_order].empty() ? -1 : l_k[l_order].back().id;
+    bool l_near = l_kin >= 0 && l_st[l_op][l_kin] == 1;
+    for( Dim const & l_d : l_rows[l_op] ) l_near = l_near || ( l_d.s == 1 && dim_types[l_d.id] != ETIR_DIM_C );
+    l_far = l_far || ( !l_near && l_bytes[l_op] > 4.0e6 );
+  }
+  double const l_plain_us = plan_us( plan, l_far, l_flops, l_bytes[0] + l_bytes[1] + l_out );
+  double const l_limit_us = 0.85 * l_plain_us - 2.0;
+  // not worth planning the alternatives: the fastest kernel and one copy
+  double const l_top = dtype_left == ETIR_BF16 ? 1100.0 : ( dtype_left == ETIR_FP64 ? 50.0 : 135.0 );
+  double const l_small = std::min( l_bytes[0], l_bytes[1] );
+  if(    std::max( l_flops / ( l_top * 1e6 ), ( l_bytes[0] + l_bytes[1] + l_out ) / 3.5e6 ) + 13.0
+       + 2.0 * l_small / 2.5e6 >= l_limit_us ) {
+    return;
+  }
+
+  // the alternatives: copy the left, the right, or both
+  struct Loops {
+    std::vector< int32_t > type;
+    std::vector< int64_t > size, s[2], aux, out;
+  };
+  struct Choice { double us; bool use[2]; Loops loops; int order; int64_t pitch; };
+  Choice l_best{ l_limit_us, { false, false }, {}, 0, 0 };
+  for( int l_ch = 1; l_ch < 4; l_ch++ ) {
+    bool const l_use[2] = { ( l_ch & 1 ) != 0, ( l_ch & 2 ) != 0 };
+    bool const l_both = l_use[0] && l_use[1];
+    Choice l_c{ 0.0, { l_use[0], l_use[1] }, {}, 0, 0 };
+    // K order: that of the operand read in place, or of the larger one
+    l_c.order = l_both ? ( l_bytes[0] >= l_bytes[1] ? 0 : 1 ) : ( l_use[0] ? 1 : 0 );
+    l_c.pitch = l_both ? ( plan.K + l_vk - 1 ) / l_vk * l_vk : plan.K;
+    Loops & l_lp = l_c.loops;
+    double l_pack_bytes = 0.0;
+    std::vector< int64_t > l_packed[2];      // stride per loop of a copied operand
+    for( int l_op = 0; l_op < 2; l_op++ ) {
+      l_packed[l_op].assign( (std::size_t) num_loops, 0 );
+      int64_t l_s = 1;
+      for( std::size_t l_i = l_k[l_c.order].size(); l_i-- > 0; ) {
+        l_packed[l_op][ l_k[l_c.order][l_i].id ] = l_s;
+        l_s *= l_k[l_c.order][l_i].size;
+      }
+      l_s = l_c.pitch;
+      for( std::size_t l_i = l_rows[l_op].size(); l_i-- > 0; ) {
+        l_packed[l_op][ l_rows[l_op][l_i].id ] = l_s;
+        l_s *= l_rows[l_op][l_i].size;
+      }
+      if( l_use[l_op] ) l_pack_bytes += double( l_s ) * double( l_esz );
+    }
+    for( int64_t l_lo = 0; l_lo < num_loops; l_lo++ ) {
+      if( sizes[l_lo] <= 1 || dim_types[l_lo] == ETIR_DIM_I || dim_types[l_lo] == ETIR_DIM_J ) continue;
+      if( l_both && dim_types[l_lo] == ETIR_DIM_K ) continue;
+      l_lp.type.push_back( dim_types[l_lo] );
+      l_lp.size.push_back( sizes[l_lo] );
+      for( int l_op = 0; l_op < 2; l_op++ ) {
+        l_lp.s[l_op].push_back( l_use[l_op] ? l_packed[l_op][l_lo] : l_st[l_op][l_lo] );
+      }
+      l_lp.aux.push_back( strides_out_aux != nullptr ? strides_out_aux[l_lo] : strides_out[l_lo] );
+      l_lp.out.push_back( strides_out[l_lo] );
+    }
+    if( l_both ) {
+      // one K loop over whole vectors: the copies' padding holds zeros
+      l_lp.type.push_back( ETIR_DIM_K );
+      l_lp.size.push_back( l_c.pitch );
+      for( int l_op = 0; l_op < 2; l_op++ ) l_lp.s[l_op].push_back( 1 );
+      l_lp.aux.push_back( 0 );
+      l_lp.out.push_back( 0 );
+    }
+    ContractionPlan l_try;
+    if( plan_contraction_impl( (int64_t) l_lp.type.size(), l_lp.type.data(), l_lp.size.data(), l_lp.s[0].data(),
+                               l_lp.s[1].data(), l_lp.aux.data(), l_lp.out.data(), dtype_left, dtype_right,
+                               dtype_comp, dtype_out, ktype_first_touch, ktype_main, ktype_last_touch, allow_split,
+                               l_try, nullptr, true ) != ETIR_SUCCESS ) {
+      continue;
+    }
+    if( plan_rate( l_try, false ) == 0.0 || !in_vec( l_try.mode_a ) || !in_vec( l_try.mode_b ) ) continue;
+    // the copies: 8 us each (launch, and the gap before the kernel that reads
+    // it) and 2.5 TB/s, read and written
+    l_c.us = plan_us( l_try, false, l_flops, l_bytes[0] + l_bytes[1] + l_out ) + 8.0 * ( l_both ? 2.0 : 1.0 )
+           + 2.0 * l_pack_bytes / 2.5e6;
+    // at most 2 GiB of workspace
+    if( l_pack_bytes > double( int64_t( 1 ) << 31 ) ) continue;
+    if( l_c.us < l_best.us ) l_best = l_c;
+  }
+  if( !l_best.use[0] && !l_best.use[1] ) return;
+
+  auto l_pk = std::make_shared< PackedContraction >();
+  auto drop = [&]() {
+    release_contraction( l_pk->cont );
+    for( PermutePlan & l_p : l_pk->perm ) release_permute( l_p );
+    if( l_pk->ws != nullptr ) (void) hipFree( l_pk->ws );
+    if( l_pk->done != nullptr ) (void) hipEventDestroy( l_pk->done );
+    (void) hipGetLastError();
+  };
+  int64_t l_total = 0;
+  for( int l_op = 0; l_op < 2; l_op++ ) {
+    if( !l_best.use[l_op] ) continue;
+    l_pk->use[l_op] = true;
+    // the copy as [C and rows][K], rows l_best.pitch elements apart
+    std::vector< int64_t > l_sz, l_si, l_so;
+    int64_t l_s = 1;
+    for( std::size_t l_i = l_k[l_best.order].size(); l_i-- > 0; ) {
+      int64_t const l_id = l_k[l_best.order][l_i].id;
+      l_sz.push_back( sizes[l_id] );
+      l_si.push_back( l_st[l_op][l_id] );
+      l_so.push_back( l_s );
+      l_s *= sizes[l_id];
+    }
+    l_s = l_best.pitch;
+    for( std::size_t l_i = l_rows[l_op].size(); l_i-- > 0; ) {
+      l_sz.push_back( l_rows[l_op][l_i].size );
+      l_si.push_back( l_rows[l_op][l_i].s );
+      l_so.push_back( l_s );
+      l_s *= l_rows[l_op][l_i].size;
+    }
+    std::reverse( l_sz.begin(), l_sz.end() );
+    std::reverse( l_si.begin(), l_si.end() );
+    std::reverse( l_so.begin(), l_so.end() );
+    if( plan_permute( (int64_t) l_sz.size(), l_sz.data(), l_si.data(), l_so.data(), dtype_left, ETIR_KTYPE_COPY,
+                      l_pk->perm[l_op] ) != ETIR_SUCCESS ) {
+      drop();
+      return;
+    }
+    l_pk->offset[l_op] = l_total;
+    l_total += ( l_s * l_esz + 255 ) / 256 * 256;
+  }
+  Loops const & l_lp = l_best.loops;
+  if(    plan_contraction_impl( (int64_t) l_lp.type.size(), l_lp.type.data(), l_lp.size.data(), l_lp.s[0].data(),
+                                l_lp.s[1].data(), l_lp.aux.data(), l_lp.out.data(), dtype_left, dtype_right,
+                                dtype_comp, dtype_out, ktype_first_touch, ktype_main, ktype_last_touch, allow_split,
+                                l_pk->cont, nullptr ) != ETIR_SUCCESS
+      || hipMalloc( &l_pk->ws, (std::size_t) l_total ) != hipSuccess
+      || ( l_best.pitch != plan.K && hipMemset( l_pk->ws, 0, (std::size_t) l_total ) != hipSuccess )
+      || hipEventCreateWithFlags( &l_pk->done, hipEventDisableTiming ) != hipSuccess ) {
+    drop();
+    return;
+  }
+  plan.packed = l_pk;
+  ContractionPlan const & l_in = l_pk->cont.partial ? *l_pk->cont.partial : l_pk->cont;
+  plan.desc += std::string( " | packed" ) + ( l_best.use[0] ? " left" : "" ) + ( l_best.use[1] ? " right" : "" )
+             + ": " + tile_str( l_in.tile ) + " K=" + std::to_string( l_best.pitch ) + " "
+             + mode_str( l_in.mode_a ) + " " + mode_str( l_in.mode_b )
+             + ( l_pk->cont.split > 1 ? " S=" + std::to_string( l_pk->cont.split ) : std::string() );
+}
+
 }  // namespace
 
 int plan_contraction( int64_t            num_loops,
@@ -1080,10 +1352,16 @@ int plan_contraction( int64_t            num_loops,
                       int32_t            ktype_last_touch,
                       ContractionPlan  & plan,
                       DevicePlacement  * place ) {
-  return plan_contraction_impl( num_loops, dim_types, sizes, strides_left, strides_right, strides_out_aux,
-                                strides_out, dtype_left, dtype_right, dtype_comp, dtype_out,
-                                ktype_first_touch, ktype_main, ktype_last_touch,
-                                std::getenv( "ETIR_NO_SPLIT_K" ) == nullptr, plan, place );
+  bool const l_split = std::getenv( "ETIR_NO_SPLIT_K" ) == nullptr;
+  int l_err = plan_contraction_impl( num_loops, dim_types, sizes, strides_left, strides_right, strides_out_aux,
+                                     strides_out, dtype_left, dtype_right, dtype_comp, dtype_out,
+                                     ktype_first_touch, ktype_main, ktype_last_touch, l_split, plan, place );
+  // the allocation-free entry point has no memory for copies
+  if( l_err == ETIR_SUCCESS && place == nullptr ) {
+    try_pack( num_loops, dim_types, sizes, strides_left, strides_right, strides_out_aux, strides_out, dtype_left,
+              dtype_right, dtype_comp, dtype_out, ktype_first_touch, ktype_main, ktype_last_touch, l_split, plan );
+  }
+  return l_err;
 }
 
 void release_contraction( ContractionPlan & plan ) {
@@ -1095,6 +1373,43 @@ void release_contraction( ContractionPlan & plan ) {
     release_contraction( *plan.partial );
     plan.partial.reset();
   }
+  if( plan.packed ) {
+    release_contraction( plan.packed->cont );
+    for( PermutePlan & l_p : plan.packed->perm ) release_permute( l_p );
+    if( plan.packed->ws != nullptr ) (void) hipFree( plan.packed->ws );
+    if( plan.packed->done != nullptr ) (void) hipEventDestroy( plan.packed->done );
+    plan.packed.reset();
+  }
+}
+
+// The packed form of a contraction on `stream`.  The workspace is the plan's
+// one: an execution on another stream than the last waits for that one's end
+// (also on the per-thread default stream, whose one handle names a stream per
+// thread).
+static int launch_packed( PackedContraction & pk,
+                          void const        * left,
+                          void const        * right,
+                          void const        * out_aux,
+                          void              * out,
+                          hipStream_t         stream ) {
+  std::lock_guard< std::mutex > l_guard( pk.lock );
+  if( pk.ran && ( pk.stream != stream || stream == hipStreamPerThread ) ) {
+    ETIR_HIP_CHECK( hipStreamWaitEvent( stream, pk.done, 0 ) );
+  }
+  void const * l_op[2] = { left, right };
+  int l_err = ETIR_SUCCESS;
+  for( int l_i = 0; l_i < 2 && l_err == ETIR_SUCCESS; l_i++ ) {
+    if( !pk.use[l_i] ) continue;
+    void * l_copy = static_cast< char * >( pk.ws ) + pk.offset[l_i];
+    l_err = launch_permute( pk.perm[l_i], l_op[l_i], l_copy, stream );
+    l_op[l_i] = l_copy;
+  }
+  if( l_err == ETIR_SUCCESS ) l_err = launch_contraction( pk.cont, l_op[0], l_op[1], out_aux, out, stream );
+  // recorded after an error too: what was enqueued still uses the workspace
+  pk.ran = true;
+  pk.stream = stream;
+  ETIR_HIP_CHECK( hipEventRecord( pk.done, stream ) );
+  return l_err;
 }
 
 int launch_contraction( ContractionPlan const & plan,
@@ -1109,6 +1424,15 @@ int launch_contraction( ContractionPlan const & plan,
   }
   if( plan.needs_aux && out_aux == nullptr ) {
     return fail( ETIR_NO_DATA_PTR_PROVIDED, "contraction: touch kernel needs the auxiliary tensor" );
+  }
+  if( plan.packed ) {
+    // under stream capture the operands are read in place: replays of a graph
+    // are ordered with nothing that uses the workspace outside it
+    hipStreamCaptureStatus l_cap = hipStreamCaptureStatusNone;
+    if( hipStreamIsCapturing( stream, &l_cap ) == hipSuccess && l_cap == hipStreamCaptureStatusNone ) {
+      return launch_packed( *plan.packed, left, right, out_aux, out, stream );
+    }
+    (void) hipGetLastError();
   }
   if( plan.split > 1 ) {
     int l_err = launch_contraction( *plan.partial, left, right, nullptr, plan.d_ws, stream );

@@ -6,6 +6,7 @@
 
 #include <cstdint>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <type_traits>
 #include <vector>
@@ -296,6 +297,8 @@ struct ContractArgs {
   int32_t  panel_grid;
 };
 
+struct PackedContraction;
+
 struct ContractionPlan {
   int32_t dtype_in   = ETIR_FP32;
   int32_t dtype_comp = ETIR_FP32;
@@ -336,9 +339,27 @@ struct ContractionPlan {
   int64_t out_dense_aux = 0;
   void *  d_ws = nullptr;
   std::shared_ptr< ContractionPlan > partial;
+  // operands copied K-contiguous into a workspace first (null: read in place)
+  std::shared_ptr< PackedContraction > packed;
   // tables and workspace live in a caller's region (DevicePlacement), not in
   // memory the plan allocated and frees
   bool    placed = false;
+};
+
+// A contraction over K-contiguous copies of one or both operands (slots: 0
+// left, 1 right): two permutations into the plan's workspace, then `cont` on
+// them.  One workspace for all executions: an execution on another stream
+// than the last one waits for `done`, which every execution records.
+struct PackedContraction {
+  ContractionPlan cont;
+  PermutePlan perm[2];
+  bool        use[2] = { false, false };
+  void *      ws     = nullptr;
+  int64_t     offset[2] = { 0, 0 };     // bytes into ws
+  std::mutex  lock;
+  hipEvent_t  done   = nullptr;
+  hipStream_t stream = nullptr;         // of the last execution
+  bool        ran    = false;
 };
 
 // Where a plan's device memory comes from when it may not allocate: a

@@ -99,7 +99,10 @@ typedef struct etir_plan_s * etir_plan_t;
  * FP64 throughout.
  *
  * The plan owns small device-resident offset tables (allocated here, never
- * during execution).
+ * during execution).  Where operands that the kernels would gather element by
+ * element are large enough, it also owns K-contiguous copies of one or both
+ * (at most 2 GiB), which every execution refills; executions of one plan on
+ * different streams then take turns (ordered by an event).
  */
 int etir_hip_contraction_create( int64_t         num_loops,
                                  int32_t const * dim_types,
@@ -134,7 +137,8 @@ int etir_hip_contraction_execute( etir_plan_t  plan,
 /*
  * Plans and executes one contraction without allocating device memory: the
  * arguments of etir_hip_contraction_create followed by those of
- * etir_hip_contraction_execute, with the same results.  No counterpart in
+ * etir_hip_contraction_execute, with the same results (up to the order of the
+ * sums where a plan would copy its operands first).  No counterpart in
  * the reference: it is for callers that cannot allocate (code under stream
  * capture, tight serving loops, harnesses that forbid hipMalloc).  The
  * offset tables and any split-K workspace live in a fixed 64 MiB device

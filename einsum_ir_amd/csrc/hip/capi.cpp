@@ -132,7 +132,7 @@ int etir_hip_plan_describe( etir_plan_t plan, char * buf, int64_t len ) {
     l_s = plan->cont.desc;
   }
   else {
-    static char const * l_modes[] = { "fill", "transpose", "copy_vec", "gather", "tiled", "reg4", "rows" };
+    static char const * l_modes[] = { "fill", "transpose", "copy_vec", "gather", "tiled", "reg4", "rows", "pair" };
     etir::PermutePlan const & p = plan->perm;
     char l_tmp[256];
     std::snprintf( l_tmp, sizeof( l_tmp ), "permute %s dims=%d elems=%lld vec=%d",

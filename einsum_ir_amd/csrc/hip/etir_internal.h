@@ -50,6 +50,7 @@ enum class PermMode : int32_t {
   GATHER    = 3,  // anything else: one thread per output element
   TILED     = 4,  // small unit-stride dims: tiles over both tensors' innermost runs
   REG4      = 5,  // short unit-stride dims: 4 x 4 register transposes, 16-byte rows through LDS
+  PAIR      = 7,  // a size-2 dim interleaved on one side, planar on the other (complex tensors)
   ROWS      = 6   // shared short unit-stride dim: tiles of whole rows, both sides' runs contiguous
 };
 
@@ -102,7 +103,7 @@ struct PermArgs {
   int32_t  vec_wide;  // COPY_VEC / FILL, bf16: 8-element (16-byte) vectors allowed
   int32_t  slot_pi;   // REG4: LDS pitch (16-byte slots) of i and of c
   int32_t  slot_pc;
-  int32_t  nt_store;  // TRANSPOSE: streaming (non-temporal) output stores
+  int32_t  xcd_group; // TRANSPOSE: neighbouring tiles on one XCD (rows that are not whole 128-byte lines)
   // TRANSPOSE, 2-byte 16-byte-read tile: o1_size > 0 folds the output's
   // next dim (output stride o1_size, input stride s_in_o2) into o, which then
   // runs over o1 + o1_size * o2 (size_o = o1_size * that dim's size);
@@ -141,10 +142,12 @@ struct PermutePlan {
   int64_t  s_out[kPermMaxDims];
   PermArgs args{};                       // pointers filled at execute time
   void *   d_tables = nullptr;           // TILED: device offset tables (owned)
+  bool     pair_split = false;           // PAIR: the input is the interleaved side
   int32_t  tile_vw = 1;                  // TILED: elements per table entry (1 or 4)
   int32_t  rows_vw = 1;                  // ROWS: elements per chunk (16, 8 or 4 bytes; 1 element when unaligned)
   int32_t  tr_shape = 0;                 // TRANSPOSE: tile 64 x 64 (0), 128 x 32 (1) or 32 x 128 (2), i x o;
                                          // 2-byte elements with 16-byte reads: 128 x 64 (3), 128 x 32 (4)
+  bool     tr_lines = false;             // TRANSPOSE, COPY_VEC: output rows of whole 128-byte lines
   int64_t  rows_len = 0;                 // ROWS: row length (elements of the shared unit-stride dim)
 };
 

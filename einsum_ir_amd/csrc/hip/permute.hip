@@ -82,10 +82,12 @@ constexpr int kThreads = 256;
 // 32 x 32: 74 % of HBM peak against 58 % tiled; 24 x 32, whose 96-byte input
 // runs split lines: 47 % against 53 % tiled)
 constexpr int64_t kReg4MaxShort = 16;
-constexpr int kPermTileMax = 4096;   // elements of a TILED tile
+constexpr int kPermTileMax = 4096;   // elements of a TILED tile (512 in small tensors)
 
 // 16-byte store that does not keep the line in the caches (the output is
-// written once and not read again by the kernel)
+// written once and not read again by the kernel); other sizes plain (an fp64
+// vector as two such stores, each 16 of every 32 bytes: 2048 x 2048 14.8 ->
+// 25.2 us)
 template< typename V >
 __device__ inline void store_stream( V * p, V const & v ) {
   if constexpr( sizeof( V ) == 16 ) {
@@ -96,6 +98,12 @@ __device__ inline void store_stream( V * p, V const & v ) {
     *p = v;
   }
 }
+
+// Type of an element held between its load and its store: 2-byte elements
+// take a register each.  Packed in pairs, the second load into a register
+// waits for the first (bf16 4095 x 4095: 31 us packed, 15 us not).
+template< typename T > struct OwnReg { typedef T type; };
+template<> struct OwnReg< uint16_t > { typedef uint32_t type; };
 
 // Next digit of a workgroup index in the mixed radix of the grid: returns
 // io_rest % i_size and leaves io_rest / i_size.  Every radix is a factor of
@@ -108,6 +116,20 @@ __device__ inline int64_t grid_digit( uint32_t & io_rest, int64_t i_size ) {
   uint32_t const l_r = io_rest - l_q * l_s;
   io_rest = l_q;
   return int64_t( l_r );
+}
+
+// Tile of a workgroup: consecutive workgroups go to the 8 XCDs in turn, each
+// with an L2 of its own; here each XCD takes one contiguous range of tiles, so
+// that lines shared by neighbouring tiles (rows that are not whole 128-byte
+// lines) are completed in one L2 (fp32 abcd->dbca 100^4: 307 -> 235 us with
+// that and the batched loads).  Not for rows of whole lines: 4096 x 4096 took
+// 33.3 us that way and 31.1 with neighbours spread over the XCDs; nor for the
+// ROWS and TILED kernels (fp32 abcd->cabd 16,128,256,32: 28.7 -> 34.7 us).
+__device__ inline uint32_t xcd_tile( bool group ) {
+  if( !group ) return blockIdx.x;
+  uint32_t const l_per = gridDim.x >> 3;
+  uint32_t const l_bid = blockIdx.x;
+  return l_bid < 8 * l_per ? ( l_bid & 7 ) * l_per + ( l_bid >> 3 ) : l_bid;
 }
 
 // LDS-tiled transpose of one TI x TO (i, o) tile per workgroup (64 x 64, or
@@ -237,16 +259,27 @@ void perm_transpose16_kernel( PermArgs a ) {
   }
 }
 
-template< typename T, int TI, int TO >
+// VEC: 4 consecutive elements per access on both sides (16 bytes for fp32);
+// otherwise one element per lane, neighbours in neighbouring lanes, so that a
+// wave's access is one run of the tensor whatever its alignment (with 4
+// consecutive elements per thread loaded one by one, fp32 4095 x 4095 ran at
+// 2.7 TB/s against 4.3 at 4096: 50.5 -> 37 us; bf16 31.4 -> 15 us).  All loads of a
+// thread are issued before the first LDS store.
+// NT: streaming stores, where the output rows are whole 128-byte lines (fp32
+// abcd->dbca 64^4 over tensors not in the caches 31.1 -> 21.7 us, 4096 x 4096
+// 31.3 -> 24.6 us); lines written in two pieces are slower that way (abcd->bdac
+// 36,48,36,512: 53.9 -> 77.8 us).  A compile-time choice: behind a run-time one
+// the compiler merges both stores into a plain one.
+template< typename T, int TI, int TO, bool VEC, bool NT >
 __global__ __launch_bounds__( kThreads )
 void perm_transpose_kernel( PermArgs a ) {
-  static_assert( TI * TO == 4 * 4 * kThreads, "four passes of 4 elements per thread" );
-  constexpr int PITCH = TI + ( TI == TO ? 1 : 2 );
+  static_assert( TI * TO == 4 * 4 * kThreads, "16 elements per thread" );
+  constexpr int PITCH = VEC ? TI + ( TI == TO ? 1 : 2 ) : TI + ( TI == 128 ? 2 : 1 );
   constexpr int RT = TI / 4;              // read: threads per o row
   constexpr int WT = TO / 4;              // write: threads per i row
   __shared__ T l_tile[TO][PITCH];
 
-  uint32_t l_bid = blockIdx.x;
+  uint32_t l_bid = xcd_tile( a.xcd_group != 0 );
   int64_t const l_ti = grid_digit( l_bid, a.tiles_i );
   int64_t const l_to = grid_digit( l_bid, a.tiles_o );
 
@@ -264,71 +297,81 @@ void perm_transpose_kernel( PermArgs a ) {
   int64_t const l_i0 = l_ti * TI;
   int64_t const l_o0 = l_to * TO;
   int const l_t  = threadIdx.x;
-  int const l_c4 = l_t % RT;
-  int const l_r  = l_t / RT;
 
-  // read: rows along o, 4 consecutive i per thread
+  if constexpr( VEC ) {
+    int const l_c4 = l_t % RT;
+    int const l_r  = l_t / RT;
+    // read: rows along o, 4 consecutive i per thread (fp64 row by row: its
+    // four 32-byte vectors at once measured 1-5 % slower)
+    constexpr int NB = sizeof( T ) == 8 ? 1 : 4;
 #pragma unroll
-  for( int l_p = 0; l_p < 4; l_p++ ) {
-    int const l_row = l_r + ( kThreads / RT ) * l_p;
-    int64_t const l_o = l_o0 + l_row;
-    int64_t const l_i = l_i0 + 4 * l_c4;
-    T l_v[4] = { T(0), T(0), T(0), T(0) };
-    if( a.vec_ok ) {
-      if( l_o < a.size_o && l_i < a.size_i ) {
-        Vec4< T > l_tmp = *reinterpret_cast< Vec4< T > const * >( l_in + l_o * a.s_in_o + l_i );
+    for( int l_p0 = 0; l_p0 < 4; l_p0 += NB ) {
+      Vec4< T > l_v[NB];
 #pragma unroll
-        for( int l_e = 0; l_e < 4; l_e++ ) l_v[l_e] = l_tmp.v[l_e];
+      for( int l_p = 0; l_p < NB; l_p++ ) {
+        int64_t const l_o = l_o0 + l_r + ( kThreads / RT ) * ( l_p0 + l_p );
+        int64_t const l_i = l_i0 + 4 * l_c4;
+        if( l_o < a.size_o && l_i < a.size_i ) {
+          l_v[l_p] = *reinterpret_cast< Vec4< T > const * >( l_in + l_o * a.s_in_o + l_i );
+        }
       }
-    }
-    else {
 #pragma unroll
-      for( int l_e = 0; l_e < 4; l_e++ ) {
-        if( l_o < a.size_o && l_i + l_e < a.size_i ) {
-          l_v[l_e] = l_in[ l_o * a.s_in_o + l_i + l_e ];
+      for( int l_p = 0; l_p < NB; l_p++ ) {
+#pragma unroll
+        for( int l_e = 0; l_e < 4; l_e++ ) {
+          l_tile[l_r + ( kThreads / RT ) * ( l_p0 + l_p )][4 * l_c4 + l_e] = l_v[l_p].v[l_e];
         }
       }
     }
-#pragma unroll
-    for( int l_e = 0; l_e < 4; l_e++ ) l_tile[l_row][4 * l_c4 + l_e] = l_v[l_e];
-  }
 
-  __syncthreads();
+    __syncthreads();
 
-  // write: rows along i, 4 consecutive o per thread
-  int const l_wc4 = l_t % WT;
-  int const l_wr  = l_t / WT;
+    // write: rows along i, 4 consecutive o per thread
+    int const l_wc4 = l_t % WT;
+    int const l_wr  = l_t / WT;
 #pragma unroll
-  for( int l_p = 0; l_p < 4; l_p++ ) {
-    int const l_row = l_wr + ( kThreads / WT ) * l_p;
-    int64_t const l_i = l_i0 + l_row;
-    int64_t const l_o = l_o0 + 4 * l_wc4;
-    T l_v[4];
-#pragma unroll
-    for( int l_e = 0; l_e < 4; l_e++ ) l_v[l_e] = l_tile[4 * l_wc4 + l_e][l_row];
-
-    if( a.vec_ok ) {
+    for( int l_p = 0; l_p < 4; l_p++ ) {
+      int const l_row = l_wr + ( kThreads / WT ) * l_p;
+      int64_t const l_i = l_i0 + l_row;
+      int64_t const l_o = l_o0 + 4 * l_wc4;
       if( l_i < a.size_i && l_o < a.size_o ) {
+        Vec4< T > l_x;
+#pragma unroll
+        for( int l_e = 0; l_e < 4; l_e++ ) l_x.v[l_e] = l_tile[4 * l_wc4 + l_e][l_row];
         Vec4< T > * l_ptr = reinterpret_cast< Vec4< T > * >( l_out + l_i * a.s_out_i + l_o );
         if( a.add ) {
           Vec4< T > l_old = *l_ptr;
 #pragma unroll
-          for( int l_e = 0; l_e < 4; l_e++ ) l_v[l_e] = Elem< T >::add( l_old.v[l_e], l_v[l_e] );
+          for( int l_e = 0; l_e < 4; l_e++ ) l_x.v[l_e] = Elem< T >::add( l_old.v[l_e], l_x.v[l_e] );
         }
-        Vec4< T > l_tmp;
-#pragma unroll
-        for( int l_e = 0; l_e < 4; l_e++ ) l_tmp.v[l_e] = l_v[l_e];
-        if( a.nt_store ) store_stream( l_ptr, l_tmp );
-        else             *l_ptr = l_tmp;
+        if constexpr( NT ) store_stream( l_ptr, l_x );
+        else               *l_ptr = l_x;
       }
     }
-    else {
+  }
+  else {
+    constexpr int kPer = TI * TO / kThreads;
+    typename OwnReg< T >::type l_v[kPer];
 #pragma unroll
-      for( int l_e = 0; l_e < 4; l_e++ ) {
-        if( l_i < a.size_i && l_o + l_e < a.size_o ) {
-          T * l_ptr = l_out + l_i * a.s_out_i + l_o + l_e;
-          *l_ptr = a.add ? Elem< T >::add( *l_ptr, l_v[l_e] ) : l_v[l_e];
-        }
+    for( int l_p = 0; l_p < kPer; l_p++ ) {
+      int64_t const l_o = l_o0 + ( l_p * kThreads + l_t ) / TI;
+      int64_t const l_i = l_i0 + l_t % TI;
+      if( l_o < a.size_o && l_i < a.size_i ) l_v[l_p] = l_in[l_o * a.s_in_o + l_i];
+    }
+#pragma unroll
+    for( int l_p = 0; l_p < kPer; l_p++ ) l_tile[( l_p * kThreads + l_t ) / TI][l_t % TI] = T( l_v[l_p] );
+
+    __syncthreads();
+
+#pragma unroll
+    for( int l_p = 0; l_p < kPer; l_p++ ) {
+      int const l_row = ( l_p * kThreads + l_t ) / TO;
+      int64_t const l_i = l_i0 + l_row;
+      int64_t const l_o = l_o0 + l_t % TO;
+      if( l_i < a.size_i && l_o < a.size_o ) {
+        T * l_ptr = l_out + l_i * a.s_out_i + l_o;
+        T const l_x = l_tile[l_t % TO][l_row];
+        *l_ptr = a.add ? Elem< T >::add( *l_ptr, l_x ) : l_x;
       }
     }
   }
@@ -346,7 +389,7 @@ __device__ inline bool perm_tile_inside( uint32_t coords, uint32_t lim, int nd )
   return true;
 }
 
-template< typename T, int V >
+template< typename T, int V, int PER >
 __global__ __launch_bounds__( kThreads )
 void perm_tiled_kernel( PermArgs a ) {
   extern __shared__ __attribute__( ( aligned( 16 ) ) ) char l_lds_raw[];
@@ -379,23 +422,51 @@ void perm_tiled_kernel( PermArgs a ) {
   int const l_nv = a.tile_n / V;
   bool const l_vec = ( V > 1 ) && a.vec_ok;
 
+  // Entries go in batches of PER per thread, the loads of a batch all issued
+  // before the first is used (entries past the tile or outside it load the
+  // tile's first element): one round trip to memory per batch.  Entry by
+  // entry, a tile of 3360 elements took 13 of them one after the other
+  // (fp32 [30,24,28,2] -> [2,24,28,30], 12 workgroups: 27 us).
+  constexpr int kPer = PER;
   // read: entry j = input-order elements V j .. V j + V - 1, contiguous in the input
-  for( int l_j = threadIdx.x; l_j < l_nv; l_j += kThreads ) {
-    if( !( l_full || perm_tile_inside( uint32_t( a.tab_rc[l_j] ), l_lim, a.tile_nd ) ) ) continue;
-    int32_t const l_off = a.tab_r[l_j];
-    T l_v[V];
-    if( l_vec ) {
-      Vec4< T > const l_x = *reinterpret_cast< Vec4< T > const * >( l_in + l_off );
+  for( int l_j0 = threadIdx.x; l_j0 < l_nv; l_j0 += kPer * kThreads ) {
+    bool    l_ok[kPer];
+    int32_t l_off[kPer];
+    typename std::conditional< V == 1, typename OwnReg< T >::type, T >::type l_v[kPer][V];
 #pragma unroll
-      for( int l_q = 0; l_q < V; l_q++ ) l_v[l_q] = l_x.v[l_q];
+    for( int l_p = 0; l_p < kPer; l_p++ ) {
+      int const l_j = l_j0 + l_p * kThreads;
+      l_ok[l_p] = l_j < l_nv;
+      l_off[l_p] = a.tab_r[l_ok[l_p] ? l_j : 0];
     }
-    else {
+    if( !l_full ) {
 #pragma unroll
-      for( int l_q = 0; l_q < V; l_q++ ) l_v[l_q] = l_in[l_off + l_q];
+      for( int l_p = 0; l_p < kPer; l_p++ ) {
+        int const l_j = l_j0 + l_p * kThreads;
+        l_ok[l_p] = l_ok[l_p] && perm_tile_inside( uint32_t( a.tab_rc[l_ok[l_p] ? l_j : 0] ), l_lim, a.tile_nd );
+        if( !l_ok[l_p] ) l_off[l_p] = 0;
+      }
     }
-    int const l_t = V * l_j;
 #pragma unroll
-    for( int l_q = 0; l_q < V; l_q++ ) l_tile[l_t + l_q + ( ( l_t + l_q ) >> 6 ) * a.tile_pad] = l_v[l_q];
+    for( int l_p = 0; l_p < kPer; l_p++ ) {
+      if( l_vec ) {
+        Vec4< T > const l_x = *reinterpret_cast< Vec4< T > const * >( l_in + l_off[l_p] );
+#pragma unroll
+        for( int l_q = 0; l_q < V; l_q++ ) l_v[l_p][l_q] = l_x.v[l_q];
+      }
+      else {
+#pragma unroll
+        for( int l_q = 0; l_q < V; l_q++ ) l_v[l_p][l_q] = l_in[l_off[l_p] + l_q];
+      }
+    }
+#pragma unroll
+    for( int l_p = 0; l_p < kPer; l_p++ ) {
+      int const l_t = V * ( l_j0 + l_p * kThreads );
+      if( l_ok[l_p] ) {
+#pragma unroll
+        for( int l_q = 0; l_q < V; l_q++ ) l_tile[l_t + l_q + ( ( l_t + l_q ) >> 6 ) * a.tile_pad] = T( l_v[l_p][l_q] );
+      }
+    }
   }
   __syncthreads();
   // write: entry j = output-order elements V j .. V j + V - 1, contiguous in
@@ -403,33 +474,126 @@ void perm_tiled_kernel( PermArgs a ) {
   // others follow at tile_t_step (they differ only in the output's
   // unit-stride dim)
   int2 const * l_tw = reinterpret_cast< int2 const * >( a.tab_w );
-  for( int l_j = threadIdx.x; l_j < l_nv; l_j += kThreads ) {
-    if( !( l_full || perm_tile_inside( uint32_t( a.tab_wc[l_j] ), l_lim, a.tile_nd ) ) ) continue;
-    int2 const l_e = l_tw[l_j];
-    T l_v[V];
+  for( int l_j0 = threadIdx.x; l_j0 < l_nv; l_j0 += kPer * kThreads ) {
+    bool l_ok[kPer];
+    int2 l_e[kPer];
+    T    l_old[kPer][V];
 #pragma unroll
-    for( int l_q = 0; l_q < V; l_q++ ) {
-      int const l_t = l_e.y + l_q * a.tile_t_step;
-      l_v[l_q] = l_tile[l_t + ( l_t >> 6 ) * a.tile_pad];
+    for( int l_p = 0; l_p < kPer; l_p++ ) {
+      int const l_j = l_j0 + l_p * kThreads;
+      l_ok[l_p] = l_j < l_nv;
+      l_e[l_p] = l_tw[l_ok[l_p] ? l_j : 0];
     }
-    T * l_ptr = l_out + l_e.x;
-    if( l_vec ) {
-      Vec4< T > l_x;
-      if( a.add ) {
-        Vec4< T > const l_old = *reinterpret_cast< Vec4< T > const * >( l_ptr );
+    if( !l_full ) {
 #pragma unroll
-        for( int l_q = 0; l_q < V; l_q++ ) l_x.v[l_q] = Elem< T >::add( l_old.v[l_q], l_v[l_q] );
+      for( int l_p = 0; l_p < kPer; l_p++ ) {
+        int const l_j = l_j0 + l_p * kThreads;
+        l_ok[l_p] = l_ok[l_p] && perm_tile_inside( uint32_t( a.tab_wc[l_ok[l_p] ? l_j : 0] ), l_lim, a.tile_nd );
+        if( !l_ok[l_p] ) l_e[l_p] = make_int2( 0, 0 );
+      }
+    }
+    if( a.add ) {
+#pragma unroll
+      for( int l_p = 0; l_p < kPer; l_p++ ) {
+#pragma unroll
+        for( int l_q = 0; l_q < V; l_q++ ) l_old[l_p][l_q] = l_out[l_e[l_p].x + l_q];
+      }
+    }
+#pragma unroll
+    for( int l_p = 0; l_p < kPer; l_p++ ) {
+      if( !l_ok[l_p] ) continue;
+      T l_v[V];
+#pragma unroll
+      for( int l_q = 0; l_q < V; l_q++ ) {
+        int const l_t = l_e[l_p].y + l_q * a.tile_t_step;
+        l_v[l_q] = l_tile[l_t + ( l_t >> 6 ) * a.tile_pad];
+        if( a.add ) l_v[l_q] = Elem< T >::add( l_old[l_p][l_q], l_v[l_q] );
+      }
+      T * l_ptr = l_out + l_e[l_p].x;
+      if( l_vec ) {
+        Vec4< T > l_x;
+#pragma unroll
+        for( int l_q = 0; l_q < V; l_q++ ) l_x.v[l_q] = l_v[l_q];
+        *reinterpret_cast< Vec4< T > * >( l_ptr ) = l_x;
       }
       else {
 #pragma unroll
-        for( int l_q = 0; l_q < V; l_q++ ) l_x.v[l_q] = l_v[l_q];
+        for( int l_q = 0; l_q < V; l_q++ ) l_ptr[l_q] = l_v[l_q];
       }
-      *reinterpret_cast< Vec4< T > * >( l_ptr ) = l_x;
+    }
+  }
+}
+
+// A dim of size 2 moved between innermost and elsewhere (complex tensors,
+// interleaved <-> planar): pairs (u, p) at 2 u + p on one side and at
+// u + p s_p on the other, u one run of size_i.  SPLIT: the input is the
+// interleaved side.  Memory-bound, no LDS: a thread moves 4 consecutive u (two
+// vectors of the interleaved side, one of each plane), a workgroup kPairU.
+// Without vectors (odd runs or strides) it moves single elements, neighbours
+// in neighbouring lanes.
+constexpr int kPairU = 4 * kThreads;
+
+template< typename T, bool SPLIT >
+__global__ __launch_bounds__( kThreads )
+void perm_pair_kernel( PermArgs a ) {
+  uint32_t l_bid = blockIdx.x;
+  int64_t const l_u0 = grid_digit( l_bid, a.tiles_i ) * kPairU;
+  int64_t l_off_in = 0, l_off_out = 0;
+  for( int l_d = a.num_batch - 1; l_d >= 0; l_d-- ) {
+    int64_t const l_idx = grid_digit( l_bid, a.batch_size[l_d] );
+    l_off_in  += l_idx * a.batch_s_in[l_d];
+    l_off_out += l_idx * a.batch_s_out[l_d];
+  }
+  T const * l_in  = reinterpret_cast< T const * >( a.in ) + l_off_in;
+  T       * l_out = reinterpret_cast< T * >( a.out ) + l_off_out;
+  int64_t const l_sp = SPLIT ? a.s_out_i : a.s_in_o;   // stride between the planes
+
+  if( a.vec_ok ) {
+    int64_t const l_u = l_u0 + 4 * int64_t( threadIdx.x );
+    if( l_u >= a.size_i ) return;
+    int64_t const l_pi = SPLIT ? 2 * l_u : l_u, l_po = SPLIT ? l_u : 2 * l_u;
+    Vec4< T > const l_a = *reinterpret_cast< Vec4< T > const * >( l_in + l_pi );
+    Vec4< T > const l_b = *reinterpret_cast< Vec4< T > const * >( l_in + l_pi + ( SPLIT ? 4 : l_sp ) );
+    Vec4< T > l_x, l_y;
+    if constexpr( SPLIT ) {
+      l_x = Vec4< T >{ { l_a.v[0], l_a.v[2], l_b.v[0], l_b.v[2] } };
+      l_y = Vec4< T >{ { l_a.v[1], l_a.v[3], l_b.v[1], l_b.v[3] } };
     }
     else {
+      l_x = Vec4< T >{ { l_a.v[0], l_b.v[0], l_a.v[1], l_b.v[1] } };
+      l_y = Vec4< T >{ { l_a.v[2], l_b.v[2], l_a.v[3], l_b.v[3] } };
+    }
+    Vec4< T > * l_px = reinterpret_cast< Vec4< T > * >( l_out + l_po );
+    Vec4< T > * l_py = reinterpret_cast< Vec4< T > * >( l_out + l_po + ( SPLIT ? l_sp : 4 ) );
+    if( a.add ) {
+      Vec4< T > const l_ox = *l_px, l_oy = *l_py;
 #pragma unroll
-      for( int l_q = 0; l_q < V; l_q++ ) {
-        l_ptr[l_q] = a.add ? Elem< T >::add( l_ptr[l_q], l_v[l_q] ) : l_v[l_q];
+      for( int l_q = 0; l_q < 4; l_q++ ) {
+        l_x.v[l_q] = Elem< T >::add( l_ox.v[l_q], l_x.v[l_q] );
+        l_y.v[l_q] = Elem< T >::add( l_oy.v[l_q], l_y.v[l_q] );
+      }
+    }
+    *l_px = l_x;
+    *l_py = l_y;
+    return;
+  }
+  typename OwnReg< T >::type l_v[4][2];
+#pragma unroll
+  for( int l_q = 0; l_q < 4; l_q++ ) {
+    int64_t const l_u = l_u0 + l_q * kThreads + threadIdx.x;
+    if( l_u < a.size_i ) {
+#pragma unroll
+      for( int l_p = 0; l_p < 2; l_p++ ) l_v[l_q][l_p] = l_in[ SPLIT ? 2 * l_u + l_p : l_u + l_p * l_sp ];
+    }
+  }
+#pragma unroll
+  for( int l_q = 0; l_q < 4; l_q++ ) {
+    int64_t const l_u = l_u0 + l_q * kThreads + threadIdx.x;
+    if( l_u < a.size_i ) {
+#pragma unroll
+      for( int l_p = 0; l_p < 2; l_p++ ) {
+        T * l_ptr = l_out + ( SPLIT ? l_u + l_p * l_sp : 2 * l_u + l_p );
+        *l_ptr = a.add ? Elem< T >::add( *l_ptr, T( l_v[l_q][l_p] ) ) : T( l_v[l_q][l_p] );
       }
     }
   }
@@ -648,7 +812,7 @@ void perm_rows_kernel( PermArgs a ) {
     int32_t l_x = ( l_tid - l_y * l_rrun ) / l_g;
     int32_t l_c = l_tid - l_y * l_rrun - l_x * l_g;
     for( int32_t l_j0 = 0; l_j0 < l_n; l_j0 += kPer * kThreads ) {
-      V       l_v[kPer];
+      typename OwnReg< V >::type l_v[kPer];
       int32_t l_s[kPer];
 #pragma unroll
       for( int l_p = 0; l_p < kPer; l_p++ ) {
@@ -666,7 +830,7 @@ void perm_rows_kernel( PermArgs a ) {
       }
 #pragma unroll
       for( int l_p = 0; l_p < kPer; l_p++ ) {
-        if( l_s[l_p] >= 0 ) l_slots[l_s[l_p]] = l_v[l_p];
+        if( l_s[l_p] >= 0 ) l_slots[l_s[l_p]] = V( l_v[l_p] );
       }
     }
   }
@@ -718,7 +882,9 @@ void perm_rows_kernel( PermArgs a ) {
 // 16-byte vector for bf16 and fp32, 32 bytes for fp64).  I is the type of
 // the element index the coordinates are decoded from: uint32_t when the
 // element count fits it (32-bit division), else uint64_t.
-template< typename T, int VW, bool FILL, typename I >
+// NT: streaming stores (COPY_VEC, fp32 and bf16, of whole 128-byte lines: abc->bac
+// 64,512,1024 bf16 27.1 -> 20.8 us; 512,512,96 fp32 41.0 -> 36.5 us).
+template< typename T, int VW, bool FILL, typename I, bool NT >
 __global__ __launch_bounds__( kThreads )
 void perm_gather_kernel( PermArgs a ) {
   typedef VecN< T, VW > V;
@@ -752,7 +918,8 @@ void perm_gather_kernel( PermArgs a ) {
 #pragma unroll
       for( int l_e = 0; l_e < VW; l_e++ ) l_v.v[l_e] = Elem< T >::add( l_old.v[l_e], l_v.v[l_e] );
     }
-    *reinterpret_cast< V * >( l_out ) = l_v;
+    if constexpr( NT ) store_stream( reinterpret_cast< V * >( l_out ), l_v );
+    else               *reinterpret_cast< V * >( l_out ) = l_v;
   }
 }
 
@@ -792,12 +959,35 @@ int launch_typed( PermutePlan const & p,
       return fail( ETIR_UNDEFINED_ERROR, "permute: grid too large" );
     }
     std::size_t const l_lds = std::size_t( a.tile_n + ( a.tile_n >> 6 ) * a.tile_pad ) * sizeof( T );
+    // batches of loads: 8 entries (4 of four elements); 2-byte elements on many
+    // workgroups one by one, whose other wavefronts hide the round trips
+    // already (abcde->eabcd 16,64,64,32,16 bf16: 49.3 us, 53.1 in batches; fp32
+    // equal; abcd->dcba 24,65,63,31 fp32 27.1 us one by one, 23.8 in batches of 8)
+    auto go = [&]( auto v_c, auto per_c ) {
+      hipLaunchKernelGGL( ( perm_tiled_kernel< T, decltype( v_c )::value, decltype( per_c )::value > ),
+                          dim3( (uint32_t) l_blocks ), dim3( kThreads ), l_lds, stream, a );
+    };
+    std::integral_constant< int, 1 > const l_1{};
+    std::integral_constant< int, 4 > const l_4{};
+    std::integral_constant< int, 8 > const l_8{};
+    bool const l_one = sizeof( T ) == 2 && l_blocks >= 512;
     if( p.tile_vw == 4 ) {
-      hipLaunchKernelGGL( ( perm_tiled_kernel< T, 4 > ), dim3( (uint32_t) l_blocks ), dim3( kThreads ), l_lds, stream, a );
+      if( l_one ) go( l_4, l_1 );
+      else        go( l_4, l_4 );
     }
     else {
-      hipLaunchKernelGGL( ( perm_tiled_kernel< T, 1 > ), dim3( (uint32_t) l_blocks ), dim3( kThreads ), l_lds, stream, a );
+      if( l_one ) go( l_1, l_1 );
+      else        go( l_1, l_8 );
     }
+  }
+  else if( p.mode == PermMode::PAIR ) {
+    int64_t const l_blocks = a.tiles_i * a.num_batch_total;
+    if( l_blocks > 0x7fffffffLL ) {
+      return fail( ETIR_UNDEFINED_ERROR, "permute: grid too large" );
+    }
+    dim3 const l_g( (uint32_t) l_blocks );
+    if( p.pair_split ) hipLaunchKernelGGL( ( perm_pair_kernel< T, true  > ), l_g, dim3( kThreads ), 0, stream, a );
+    else               hipLaunchKernelGGL( ( perm_pair_kernel< T, false > ), l_g, dim3( kThreads ), 0, stream, a );
   }
   else if( p.mode == PermMode::REG4 ) {
     a.c_nblk = ( a.c_size + a.c_chunk - 1 ) / a.c_chunk;
@@ -848,13 +1038,13 @@ int launch_typed( PermutePlan const & p,
     if( p.tr_shape == 3 || p.tr_shape == 4 ) {
       if constexpr( sizeof( T ) == 2 ) {
         auto go = [&]( auto to_c, auto vec_c ) {
+          constexpr int  TO  = decltype( to_c )::value;
+          constexpr bool VEC = decltype( vec_c )::value;
           if( a.o1_size > 0 ) {
-            hipLaunchKernelGGL( ( perm_transpose16_kernel< T, 128, decltype( to_c )::value, decltype( vec_c )::value,
-                                                           true > ), l_g, dim3( kThreads ), 0, stream, a );
+            hipLaunchKernelGGL( ( perm_transpose16_kernel< T, 128, TO, VEC, true > ), l_g, dim3( kThreads ), 0, stream, a );
           }
           else {
-            hipLaunchKernelGGL( ( perm_transpose16_kernel< T, 128, decltype( to_c )::value, decltype( vec_c )::value,
-                                                           false > ), l_g, dim3( kThreads ), 0, stream, a );
+            hipLaunchKernelGGL( ( perm_transpose16_kernel< T, 128, TO, VEC, false > ), l_g, dim3( kThreads ), 0, stream, a );
           }
         };
         std::integral_constant< int, 64 > const l_to64{};
@@ -872,9 +1062,17 @@ int launch_typed( PermutePlan const & p,
         return fail( ETIR_UNDEFINED_ERROR, "permute: 16-byte transpose tile for a non-2-byte type" );
       }
     }
-    else if( p.tr_shape == 1 ) hipLaunchKernelGGL( ( perm_transpose_kernel< T, 128, 32 > ), l_g, dim3( kThreads ), 0, stream, a );
-    else if( p.tr_shape == 2 ) hipLaunchKernelGGL( ( perm_transpose_kernel< T, 32, 128 > ), l_g, dim3( kThreads ), 0, stream, a );
-    else                       hipLaunchKernelGGL( ( perm_transpose_kernel< T, 64, 64 > ), l_g, dim3( kThreads ), 0, stream, a );
+    else {
+      auto go = [&]( auto vec_c, auto nt_c ) {
+        constexpr bool VEC = decltype( vec_c )::value, NT = decltype( nt_c )::value;
+        if(      p.tr_shape == 1 ) hipLaunchKernelGGL( ( perm_transpose_kernel< T, 128, 32, VEC, NT > ), l_g, dim3( kThreads ), 0, stream, a );
+        else if( p.tr_shape == 2 ) hipLaunchKernelGGL( ( perm_transpose_kernel< T, 32, 128, VEC, NT > ), l_g, dim3( kThreads ), 0, stream, a );
+        else                       hipLaunchKernelGGL( ( perm_transpose_kernel< T, 64, 64, VEC, NT > ), l_g, dim3( kThreads ), 0, stream, a );
+      };
+      if( !a.vec_ok )         go( std::false_type(), std::false_type() );
+      else if( p.tr_lines && sizeof( T ) == 4 ) go( std::true_type(), std::true_type() );
+      else                    go( std::true_type(), std::false_type() );
+    }
   }
   else {
     // bf16 moves 8 elements (16 bytes) per vector where the planner allows it
@@ -887,9 +1085,13 @@ int launch_typed( PermutePlan const & p,
     auto launch = [&]( auto i_fill, auto i_idx ) {
       constexpr bool l_fill = decltype( i_fill )::value;
       typedef typename decltype( i_idx )::type I;
-      if( l_vw == 8 )      hipLaunchKernelGGL( ( perm_gather_kernel< T, 8, l_fill, I > ), l_g, dim3( kThreads ), 0, stream, a );
-      else if( l_vw == 4 ) hipLaunchKernelGGL( ( perm_gather_kernel< T, 4, l_fill, I > ), l_g, dim3( kThreads ), 0, stream, a );
-      else                 hipLaunchKernelGGL( ( perm_gather_kernel< T, 1, l_fill, I > ), l_g, dim3( kThreads ), 0, stream, a );
+      constexpr int l_wide = sizeof( T ) == 2 ? 8 : 4;
+      if( !l_fill && l_vw == l_wide && p.tr_lines && sizeof( T ) <= 4 ) {
+        hipLaunchKernelGGL( ( perm_gather_kernel< T, l_wide, l_fill, I, true > ), l_g, dim3( kThreads ), 0, stream, a );
+      }
+      else if( l_vw == 8 ) hipLaunchKernelGGL( ( perm_gather_kernel< T, 8, l_fill, I, false > ), l_g, dim3( kThreads ), 0, stream, a );
+      else if( l_vw == 4 ) hipLaunchKernelGGL( ( perm_gather_kernel< T, 4, l_fill, I, false > ), l_g, dim3( kThreads ), 0, stream, a );
+      else                 hipLaunchKernelGGL( ( perm_gather_kernel< T, 1, l_fill, I, false > ), l_g, dim3( kThreads ), 0, stream, a );
     };
     bool const l_small = a.num_elements <= int64_t( UINT32_MAX );
     if( p.mode == PermMode::FILL ) {
@@ -1099,13 +1301,17 @@ bool plan_tiled( PermutePlan & plan, int dim_i, int dim_o ) {
     for( int64_t l_x : l_e ) l_t *= l_x;
     return l_t;
   };
+  // small tensors in smaller tiles, about two per CU: with 4096-element tiles
+  // a few CUs worked through four round trips to memory each while the
+  // others had nothing
+  int64_t const l_tile_max = std::max< int64_t >( 512, std::min< int64_t >( kPermTileMax, plan.num_elements / 512 ) );
   // tiles of kPermTileMax elements where the dims allow (grow the outermost
   // run dims): small tiles leave each workgroup too little work
   // first the run needs alone may exceed the limit: halve the largest extent,
   // the unit-stride dims' last (their multiples of 4 keep 16-byte accesses)
   int const l_ui = (int) ( std::find( l_td.begin(), l_td.end(), dim_i ) - l_td.begin() );
   int const l_uo = (int) ( std::find( l_td.begin(), l_td.end(), dim_o ) - l_td.begin() );
-  while( tile_n() > kPermTileMax ) {
+  while( tile_n() > l_tile_max ) {
     int l_big = -1;
     for( int l_k = 0; l_k < l_nt; l_k++ ) {
       if( l_k == l_ui || l_k == l_uo || l_e[l_k] <= 1 ) continue;
@@ -1122,7 +1328,7 @@ bool plan_tiled( PermutePlan & plan, int dim_i, int dim_o ) {
     for( int l_k = l_nt - 1; l_k >= 0; l_k-- ) {
       int64_t const l_cap = std::min< int64_t >( plan.size[l_td[l_k]], 128 );
       int64_t const l_new = std::min( l_cap, 2 * l_e[l_k] );
-      if( l_new > l_e[l_k] && tile_n() / l_e[l_k] * l_new <= kPermTileMax ) {
+      if( l_new > l_e[l_k] && tile_n() / l_e[l_k] * l_new <= l_tile_max ) {
         l_e[l_k] = l_new;
         l_grew = true;
       }
@@ -1397,6 +1603,14 @@ int plan_permute( int64_t         num_dims,
     }
     return true;
   };
+  // output rows along dim d are whole 128-byte lines
+  auto whole_lines = [&]( int d ) {
+    bool l_ok = ( plan.size[d] * plan.elem_bytes ) % 128 == 0;
+    for( int l_di = 0; l_di < l_n; l_di++ ) {
+      l_ok = l_ok && ( l_di == d || ( plan.s_out[l_di] * plan.elem_bytes ) % 128 == 0 );
+    }
+    return l_ok;
+  };
   // the output dim that continues the output's run after dim dof (output
   // stride = dof's size), not the input's unit-stride dim di; -1 if none
   auto fold_dim = [&]( int di, int dof ) {
@@ -1425,6 +1639,37 @@ int plan_permute( int64_t         num_dims,
     a.vec_wide = ( a.vec_ok && plan.elem_bytes == 2 && plan.size[l_n-1] % 8 == 0 );
     for( int l_di = 0; l_di < l_n - 1 && a.vec_wide; l_di++ ) {
       if( plan.s_out[l_di] % 8 != 0 ) a.vec_wide = 0;
+    }
+    return ETIR_SUCCESS;
+  }
+
+  // a dim p of size 2 innermost on one side, on the other side not, and a
+  // dim u next to it that is unit-stride there: pairs (interleaved <-> planar
+  // complex tensors), runs of at least 64
+  for( int l_p = 0; l_p < l_n; l_p++ ) {
+    if( plan.size[l_p] != 2 || ( plan.s_in[l_p] == 1 ) == ( plan.s_out[l_p] == 1 ) ) continue;
+    bool const l_split = plan.s_in[l_p] == 1;
+    int64_t const * l_si = l_split ? plan.s_in : plan.s_out;    // the interleaved side
+    int64_t const * l_sl = l_split ? plan.s_out : plan.s_in;
+    int l_u = -1;
+    for( int l_di = 0; l_di < l_n; l_di++ ) if( l_di != l_p && l_si[l_di] == 2 && l_sl[l_di] == 1 ) l_u = l_di;
+    if( l_u < 0 || plan.size[l_u] < kTile ) continue;
+    plan.mode = PermMode::PAIR;
+    plan.pair_split = l_split;
+    a.size_i  = plan.size[l_u];
+    a.s_out_i = plan.s_out[l_p];
+    a.s_in_o  = plan.s_in[l_p];
+    a.tiles_i = ( a.size_i + kPairU - 1 ) / kPairU;
+    a.vec_ok  = ( a.size_i % 4 == 0 && l_sl[l_p] % 4 == 0 ) ? 1 : 0;
+    a.num_batch_total = 1;
+    for( int l_di = 0; l_di < l_n; l_di++ ) {
+      if( l_di == l_p || l_di == l_u ) continue;
+      a.batch_size[a.num_batch]  = plan.size[l_di];
+      a.batch_s_in[a.num_batch]  = plan.s_in[l_di];
+      a.batch_s_out[a.num_batch] = plan.s_out[l_di];
+      a.num_batch_total *= plan.size[l_di];
+      a.num_batch++;
+      if( plan.s_in[l_di] % 4 != 0 || plan.s_out[l_di] % 4 != 0 ) a.vec_ok = 0;
     }
     return ETIR_SUCCESS;
   }
@@ -1712,7 +1957,9 @@ int plan_permute( int64_t         num_dims,
     a.vec_ok = (    a.size_i % 4 == 0 && a.size_o % 4 == 0
                  && a.s_in_o % 4 == 0 && a.s_out_i % 4 == 0
                  && all_div4( l_dim_i, l_dim_o ) ) ? 1 : 0;
-    a.nt_store = 1;
+    plan.tr_lines = whole_lines( l_dim_o );
+    a.xcd_group = (    ( a.size_i * plan.elem_bytes ) % 128 != 0 || ( a.size_o * plan.elem_bytes ) % 128 != 0 )
+               && a.tiles_i * a.tiles_o * a.num_batch_total >= 2048;
     return ETIR_SUCCESS;
   }
 
@@ -1728,6 +1975,7 @@ int plan_permute( int64_t         num_dims,
     plan.mode = PermMode::COPY_VEC;
     a.vec_ok = 1;
     a.vec_wide = ( plan.elem_bytes == 2 && plan.size[l_n-1] % 8 == 0 && all_div( 8, l_n - 1, l_n - 1 ) ) ? 1 : 0;
+    plan.tr_lines = whole_lines( l_n - 1 );
   }
   else {
     plan.mode = PermMode::GATHER;

@@ -482,3 +482,35 @@ def test_permute_padded_shared_unit_dim(torch_cuda, oracle, pad):
     plan.close()
     np.testing.assert_array_equal(do.cpu().numpy(), ref, err_msg=desc)
     assert ("rows" in desc) == (pad == 0), desc
+
+
+@pytest.mark.parametrize("dtype", [eir.FP32, eir.FP64, eir.BF16])
+@pytest.mark.parametrize("expr,sizes", [
+    ("abx->xab", dict(a=5, b=64, x=2)),            # one run of 320
+    ("abx->xab", dict(a=7, b=1031, x=2)),          # odd run: single elements, seven workgroups and a rest
+    ("xab->abx", dict(a=4, b=1025, x=2)),
+    ("xab->abx", dict(a=3, b=21, x=2)),            # 63: below the kernel's shortest run
+    ("abx->axb", dict(a=9, b=68, x=2)),            # batches, vectors
+    ("axb->abx", dict(a=9, b=67, x=2)),            # batches, odd strides
+    ("cabx->axcb", dict(a=3, b=65, c=4, x=2)),     # batch dims in another order
+])
+def test_pairs(torch_cuda, oracle, expr, sizes, dtype):
+    """A dim of size 2 between innermost and elsewhere (interleaved and planar
+    complex tensors), COPY and ADD."""
+    for ktype in ([eir.COPY] if dtype == eir.BF16 else [eir.COPY, eir.ADD]):
+        _check(torch_cuda, oracle, expr, sizes, dtype=dtype, ktype=ktype)
+
+
+@pytest.mark.parametrize("dtype", [eir.FP32, eir.FP64, eir.BF16])
+@pytest.mark.parametrize("expr,sizes", [
+    ("ab->ba", dict(a=65, b=127)),                 # one past a tile, one short of two
+    ("ab->ba", dict(a=2047, b=4099)),              # tiles grouped by XCD, grid no multiple of 8
+    ("abc->cba", dict(a=33, b=3, c=131)),          # 128 x 32 tiles
+    ("abc->cba", dict(a=131, b=3, c=33)),          # 32 x 128 tiles
+    ("abcd->dbca", dict(a=100, b=12, c=20, d=100)),  # vectors, rows that split lines, grouped
+    ("abcd->dcba", dict(a=23, b=17, c=33, d=61)),  # tiled, small tiles
+    ("abcd->dbca", dict(a=17, b=65, c=63, d=19)),  # tiled, more tiles than one batch of loads
+])
+def test_odd_transposes(torch_cuda, oracle, expr, sizes, dtype):
+    for ktype in ([eir.COPY] if dtype == eir.BF16 else [eir.COPY, eir.ADD]):
+        _check(torch_cuda, oracle, expr, sizes, dtype=dtype, ktype=ktype)

@@ -23,6 +23,23 @@ int launch_bf16_dma_256x128( int32_t ma, int32_t mb, ContractArgs const & a, uin
   return fail( ETIR_COMPILATION_FAILED, "no 256x128 direct-to-LDS kernel for this load-mode combination" );
 }
 
+// 128 x 128 tiles of four 64 x 64 waves, two workgroups per CU (64 KB of LDS each)
+int launch_bf16_dma_128x128( int32_t ma, int32_t mb, ContractArgs const & a, uint32_t grid, hipStream_t stream ) {
+  auto go = [&]( auto ma_c, auto mb_c ) {
+    hipLaunchKernelGGL( ( kern::contract_dma_kernel< 128, 128, 64, 2, 2, decltype( ma_c )::value,
+                                                     decltype( mb_c )::value, 2, 2 > ),
+                        dim3( grid ), dim3( 256 ), 0, stream, a );
+    return int( ETIR_SUCCESS );
+  };
+  typedef std::integral_constant< int32_t, LOAD_VEC_MN > Mn;
+  typedef std::integral_constant< int32_t, LOAD_VEC_K >  Kc;
+  if( ma == LOAD_VEC_MN && mb == LOAD_VEC_MN ) return go( Mn{}, Mn{} );
+  if( ma == LOAD_VEC_MN && mb == LOAD_VEC_K )  return go( Mn{}, Kc{} );
+  if( ma == LOAD_VEC_K  && mb == LOAD_VEC_MN ) return go( Kc{}, Mn{} );
+  if( ma == LOAD_VEC_K  && mb == LOAD_VEC_K )  return go( Kc{}, Kc{} );
+  return fail( ETIR_COMPILATION_FAILED, "no 128x128 direct-to-LDS kernel for this load-mode combination" );
+}
+
 // CUs of the current device (one persistent workgroup each)
 uint32_t device_cus() {
   int l_dev = 0;
@@ -39,6 +56,7 @@ uint32_t device_cus() {
 int launch_contract_bf16_dma( int32_t ma, int32_t mb, int32_t variant, ContractArgs const & a,
                               uint32_t grid, hipStream_t stream ) {
   if( variant == 2 ) return launch_bf16_dma_256x128( ma, mb, a, grid, stream );
+  if( variant == 4 ) return launch_bf16_dma_128x128( ma, mb, a, grid, stream );
   if( variant == 3 && ma == LOAD_VEC_MN && mb == LOAD_VEC_MN && kern::persistent_dma_eligible( a, 256, 256 ) ) {
     static thread_local int s_dev = -1;
     static thread_local uint32_t s_cus = 256;

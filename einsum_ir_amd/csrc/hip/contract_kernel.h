@@ -627,6 +627,54 @@ __device__ __attribute__( ( always_inline ) ) inline void epilogue_fast_f32(
   } );
 }
 
+// Plain bf16 output whose columns run unit-stride in aligned groups of 8: each
+// 32-row slab of a wave goes through its LDS slab, a lane reads 8 consecutive
+// columns, rounds them (v_cvt_pk_bf16_f32, to nearest even) and stores 16
+// bytes.  One element per lane and store, with a software rounding, cost more
+// than the main loop of a K of 2048: km,kn->mn 4096 a side 187 -> 136 us
+template< int TM, int TN, int PITCH >
+__device__ __attribute__( ( always_inline ) ) inline void epilogue_bf16_v8(
+    uint16_t * l_base, f32x16 const ( &l_acc )[TM][TN], float * l_slab, int32_t const * l_s_m_out,
+    int32_t const * l_s_n_out, int l_row0, int l_col0, int l_lane, int l_rows, int l_cols, bool l_relu ) {
+  typedef float  f32x2  __attribute__( ( ext_vector_type( 2 ) ) );
+  typedef __bf16 bf16x2 __attribute__( ( ext_vector_type( 2 ) ) );
+  constexpr int LPR = TN * 32 / 8;          // lanes per row
+  constexpr int RPI = 64 / LPR;             // rows per store instruction
+  int const l_lr = l_lane & 31;
+  int const l_lg = l_lane >> 5;
+  int const l_nl = l_col0 + 8 * ( l_lane % LPR );
+  bool const l_nok = l_nl < l_cols;         // groups of 8 columns are inside the tensor or outside it
+  int64_t const l_noff = l_s_n_out[l_nl];
+#pragma unroll
+  for( int l_i = 0; l_i < TM; l_i++ ) {
+    // the slab's previous reads were issued earlier by this wave, and LDS
+    // executes one wave's accesses in order
+#pragma unroll
+    for( int l_j = 0; l_j < TN; l_j++ )
+#pragma unroll
+      for( int l_r = 0; l_r < 16; l_r++ )
+        l_slab[( 8 * ( l_r >> 2 ) + 4 * l_lg + ( l_r & 3 ) ) * PITCH + l_j * 32 + l_lr] = l_acc[l_i][l_j][l_r];
+#pragma unroll
+    for( int l_q = 0; l_q < 32 / RPI; l_q++ ) {
+      int const l_row = l_q * RPI + l_lane / LPR;
+      int const l_ml  = l_row0 + l_i * 32 + l_row;
+      f32x4 const * l_p = reinterpret_cast< f32x4 const * >( l_slab + l_row * PITCH + 8 * ( l_lane % LPR ) );
+      f32x4 const l_v[2] = { l_p[0], l_p[1] };
+      u32x4 l_o;
+#pragma unroll
+      for( int l_e = 0; l_e < 4; l_e++ ) {
+        f32x2 l_x = { l_v[l_e / 2][2 * ( l_e & 1 )], l_v[l_e / 2][2 * ( l_e & 1 ) + 1] };
+        if( l_relu ) {
+          l_x[0] = fmaxf( l_x[0], 0.0f );
+          l_x[1] = fmaxf( l_x[1], 0.0f );
+        }
+        l_o[l_e] = __builtin_bit_cast( uint32_t, __builtin_convertvector( l_x, bf16x2 ) );
+      }
+      if( l_nok && l_ml < l_rows ) *reinterpret_cast< u32x4 * >( l_base + l_noff + l_s_m_out[l_ml] ) = l_o;
+    }
+  }
+}
+
 // The epilogue's output/aux offsets of the tile rows and columns, loaded into
 // registers when the workgroup starts (the loads complete under the main loop
 // instead of adding a memory round trip after it) and staged in LDS at the
@@ -730,6 +778,16 @@ __device__ __attribute__( ( always_inline ) ) inline void epilogue( ContractArgs
     };
     if( a.last_touch == ETIR_KTYPE_RELU ) store_part( std::true_type() );
     else                                  store_part( std::false_type() );
+    return;
+  }
+
+  if(    a.out_v8 && a.first_touch == ETIR_KTYPE_ZERO
+      && ( a.last_touch == ETIR_KTYPE_UNDEFINED || a.last_touch == ETIR_KTYPE_RELU ) ) {
+    uint16_t * l_base = reinterpret_cast< uint16_t * >( a.out ) + l_coff_out;
+    float * l_slab = reinterpret_cast< float * >( lds + L::TABS + ( l_wm * WN + l_wn ) * L::SLAB );
+    epilogue_bf16_v8< TM, TN, L::PITCH >( l_base, l_acc, l_slab, l_s_m_out, l_s_n_out, l_row0, l_col0, l_lane,
+                                          int( a.M - l_m0 ), int( a.N - l_n0 ),
+                                          a.last_touch == ETIR_KTYPE_RELU );
     return;
   }
 

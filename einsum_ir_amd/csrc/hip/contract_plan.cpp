@@ -154,6 +154,7 @@ char const * tile_str( int32_t t ) {
     case TILE_BF16_256x128: return "bf16_256x128x32";
     case TILE_BF16_DMA_256x256: return "bf16_dma_256x256";
     case TILE_BF16_DMA_256x128: return "bf16_dma_256x128";
+    case TILE_BF16_DMA_128x128: return "bf16_dma_128x128";
     case TILE_BF16_128x128: return "bf16_128x128x64";
     case TILE_BF16_64x64:   return "bf16_64x64x64";
     case TILE_F64_64x64:    return "f64_64x64x16";
@@ -179,6 +180,7 @@ void tile_shape( int32_t t, int64_t & bm, int64_t & bn ) {
     case TILE_F32_KWAVE_32x32: bm = 32; bn = 32; break;
     case TILE_BF16_128x128: bm = 128; bn = 128; break;
     case TILE_F32_DMA_128x128: bm = 128; bn = 128; break;
+    case TILE_BF16_DMA_128x128: bm = 128; bn = 128; break;
     default:                bm = 64;  bn = 64;  break;
   }
 }
@@ -476,7 +478,23 @@ int plan_contraction_impl( int64_t            num_loops,
       && 2 * ( max_of( l_tn_b ) + std::max< int64_t >( l_size_k - 1, 0 ) * l_sk_b ) + 64 < ( int64_t( 1 ) << 31 )
       && 2 * int64_t( 64 ) * std::max( l_sk_a, l_sk_b ) * ( ( l_size_k + 63 ) / 64 + 4 ) < ( int64_t( 1 ) << 31 );
   plan.tile_fallback = plan.tile;
-  if( l_dma_ok && n_tiles( TILE_BF16_DMA_256x256 ) >= l_cus ) plan.tile = TILE_BF16_DMA_256x256;
+  // 256 x 256 tiles where their persistent scheduled loop runs (both operands
+  // row-contiguous, whole tiles, plain fp32 output in 32-column runs: 4096 a
+  // side 109 us); everything else with a 128 x 128 tile per CU takes those,
+  // two workgroups per CU, against the generic 256 x 256 loop (one) and the
+  // register-staged tiles: mk,nk->mn 4096 a side 168 -> 126 us, 8192 x 1024 x
+  // 4096 82 -> 66 us, 4072 x 2048 x 2048 44 -> 38 us, 2304 x 2304 x 1024 20 ->
+  // 18 us; bf16 results (16-byte stores) 55 -> 36 us at 4072 x 2048 x 2048
+  std::size_t l_run_n = 1;
+  while( l_run_n < l_tn_out.size() && l_tn_out[l_run_n] == l_tn_out[l_run_n - 1] + 1 ) l_run_n++;
+  bool const l_persistent =
+         plan.mode_a == LOAD_VEC_MN && plan.mode_b == LOAD_VEC_MN && dtype_out == ETIR_FP32
+      && ktype_first_touch == ETIR_KTYPE_ZERO && ktype_last_touch == ETIR_KTYPE_UNDEFINED
+      && l_kern_m % 256 == 0 && l_kern_n % 256 == 0 && l_run_n >= 32
+      && ( l_run_n % 32 == 0 || l_run_n == l_tn_out.size() )
+      && 4 * ( max_of( l_tm_out ) + max_of( l_tn_out ) ) + 4 < ( int64_t( 1 ) << 32 );
+  if( l_dma_ok && l_persistent && n_tiles( TILE_BF16_DMA_256x256 ) >= l_cus ) plan.tile = TILE_BF16_DMA_256x256;
+  else if( l_dma_ok && n_tiles( TILE_BF16_DMA_128x128 ) >= l_cus ) plan.tile = TILE_BF16_DMA_128x128;
   // the fp32 direct-to-LDS kernel: where the planner chose the 128 x 128 fp32
   // tile, under the same conditions (4-byte elements; the loads of the step
   // past the last one are issued too); a K that is not affine up to 1024,
@@ -993,6 +1011,8 @@ int plan_contraction_impl( int64_t            num_loops,
   a.first_touch = ktype_first_touch;
   a.last_touch  = ktype_last_touch;
   a.out_bf16 = ( dtype_out == ETIR_BF16 ) ? 1 : 0;
+  a.out_v8 = ( dtype_out == ETIR_BF16 && runs_contiguous( l_tn_out, 8, 8 ) && all_multiple( l_tm_out, 8 )
+               && all_multiple( l_tc_out, 8 ) ) ? 1 : 0;
   // start-time stagger of the persistent direct-to-LDS kernel: 4 phases, 3
   // units (~3 us) apart (measured on config 3; diagnostic override by env)
   a.dma_phases = 4;
@@ -1089,6 +1109,7 @@ double plan_rate( ContractionPlan const & plan, bool far ) {
     case TILE_F32_128x128:      return by_mode( 112.0, 75.0, 75.0, 16.0 );
     case TILE_F32_64x64:        return by_mode( 65.0, 30.0, 25.0, 25.0 );
     case TILE_BF16_DMA_256x256: return plan.mode_a == LOAD_VEC_MN && plan.mode_b == LOAD_VEC_MN ? 1100.0 : 800.0;
+    case TILE_BF16_DMA_128x128: return 850.0;
     case TILE_BF16_256x128:     return by_mode( 550.0, 100.0, 95.0, 20.0 );
     case TILE_BF16_128x128:     return by_mode( 550.0, 50.0, 45.0, 20.0 );
     case TILE_BF16_64x64:       return by_mode( 300.0, 46.0, 45.0, 25.0 );
@@ -1474,6 +1495,7 @@ int launch_contraction( ContractionPlan const & plan,
   a.aux = plan.needs_aux ? out_aux : nullptr;
   a.out = out;
 
+  if( uintptr_t( out ) % 16 != 0 ) a.out_v8 = 0;
   // vector paths need aligned base pointers; otherwise fall back to gathers
   int32_t l_ma = plan.mode_a;
   int32_t l_mb = plan.mode_b;
@@ -1488,7 +1510,7 @@ int launch_contraction( ContractionPlan const & plan,
   int32_t l_dma_variant = plan.dma_variant;
   int32_t l_tile = plan.tile;
   if(    ( l_tile == TILE_BF16_DMA_256x256 || l_tile == TILE_BF16_DMA_256x128 || l_tile == TILE_F32_KWAVE_32x32
-           || l_tile == TILE_F32_DMA_128x128 )
+           || l_tile == TILE_F32_DMA_128x128 || l_tile == TILE_BF16_DMA_128x128 )
       && ( l_ma != plan.mode_a || l_mb != plan.mode_b ) ) {
     // the DMA and K-over-waves kernels need the 16-byte vector modes: use
     // the register-staged kernel with its own tile grid
@@ -1526,6 +1548,9 @@ int launch_contraction( ContractionPlan const & plan,
       break;
     case TILE_BF16_DMA_256x128:
       l_err = launch_contract_bf16_dma( l_ma, l_mb, 2, a, l_g, stream );
+      break;
+    case TILE_BF16_DMA_128x128:
+      l_err = launch_contract_bf16_dma( l_ma, l_mb, 4, a, l_g, stream );
       break;
     case TILE_F32_DMA_128x128:
       l_err = launch_contract_f32_dma( l_ma, l_mb, a, l_g, stream );

@@ -239,6 +239,7 @@ enum TileCfg : int32_t {
   TILE_F32_DMA_128x128  = 12, // fp32 direct-to-LDS kernel (contract_f32_dma.hip)
   TILE_GEMV             = 13, // M == 1 or N == 1: one thread per output element (contract_gemv.hip)
   TILE_SKINNY           = 14, // one free side of 2-64: one thread per long index (contract_skinny.hip)
+  TILE_BF16_DMA_128x128 = 16, // bf16 direct-to-LDS kernel, two workgroups per CU, any pairing of the vector modes
   TILE_PANEL            = 15  // short K, one free side of 65-256 resident in LDS (contract_panel.hip)
 };
 
@@ -270,6 +271,7 @@ struct ContractArgs {
   int32_t last_touch;     // ETIR_KTYPE_{RELU,ADD,UNDEFINED}
   int32_t k_full;         // K % BK == 0: no K masking needed
   int32_t out_bf16;       // output stored as bf16 (RNE)
+  int32_t out_v8;         // bf16 output in aligned groups of 8 unit-stride columns: 16-byte stores
   int32_t out_off32;      // every output byte offset (M part + N part, C part excluded) is < 2^32
   int32_t c_inner;        // workgroup ids walk C fastest (the output's unit-stride dim is a C dim)
   int32_t out_nt;         // output columns run in 32-element unit-stride groups: non-temporal stores

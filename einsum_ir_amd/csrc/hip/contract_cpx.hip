@@ -107,6 +107,19 @@ void contract_cpx_kernel( ContractArgs a ) {
       l_im[l_i][l_j] = V( T( 0 ) );
     }
 
+  // the output offsets of this lane's rows and columns, read here (clamped)
+  // under the main loop: read between the epilogue's stores, each waited for
+  // every store before it (one vector-memory counter for loads and stores)
+  int32_t l_mo[2][4], l_no[2];
+#pragma unroll
+  for( int l_i = 0; l_i < 2; l_i++ ) {
+    l_no[l_i] = a.tn_out[min( l_n0 + l_wn * 32 + l_i * 16 + l_r16, a.N - 1 )];
+#pragma unroll
+    for( int l_r = 0; l_r < 4; l_r++ ) {
+      l_mo[l_i][l_r] = a.tm_out[min( l_m0 + l_wm * 32 + l_i * 16 + MF::row( l_r, l_g ), a.M - 1 )];
+    }
+  }
+
   auto load = [&]( int32_t k0 ) __attribute__( ( always_inline ) ) {
     l_ld_ar.template load< KAFF >( l_a_re, k0, a.K, a.tk_a, a.sk_a );
     l_ld_ai.template load< KAFF >( l_a_im, k0, a.K, a.tk_a, a.sk_a );
@@ -165,14 +178,13 @@ void contract_cpx_kernel( ContractArgs a ) {
   for( int l_j = 0; l_j < 2; l_j++ ) {
     int32_t const l_n = l_n0 + l_wn * 32 + l_j * 16 + l_r16;
     if( l_n >= a.N ) continue;
-    int64_t const l_no = a.tn_out[l_n];
 #pragma unroll
     for( int l_i = 0; l_i < 2; l_i++ ) {
 #pragma unroll
       for( int l_r = 0; l_r < 4; l_r++ ) {
         int32_t const l_m = l_m0 + l_wm * 32 + l_i * 16 + MF::row( l_r, l_g );
         if( l_m >= a.M ) continue;
-        int64_t const l_off = int64_t( a.tm_out[l_m] ) + l_no;
+        int64_t const l_off = int64_t( l_mo[l_i][l_r] ) + l_no[l_j];
         T l_vr = l_re[l_i][l_j][l_r];
         T l_vi = l_im[l_i][l_j][l_r];
         if( l_acc_out ) {

@@ -375,6 +375,147 @@ void contract_f32_dma_kernel( ContractArgs a ) {
   epilogue< BM, BN, WM, WN, TM, TN, T >( a, l_acc, l_tabs, l_lds, l_c, l_m0, l_n0, l_wm, l_wn, l_lane );
 }
 
+// A K of one step (up to 32), plain fp32 output: one LDS stage and no slabs for
+// touch kernels, so four workgroups of 8 waves per CU.  Such a tile is one load
+// round trip, 16 MFMAs per wave and its stores, and with two workgroups per CU
+// the store queue ran dry between them (dega,gfbc->abcdef 24,20,20,24,20,20,24,
+// 369 MB of output, both operands packed: 95 us against 107-110).
+//
+// Output of short unit-stride column runs (R = 8 to 28 columns) whose rows are
+// neighbours in memory, as a tensor of many small modes has them: column by
+// column a store instruction writes pieces of 4 R bytes, and a tile edge cuts
+// a run in two.  A tile then takes whole runs (n_step columns of the 128), is
+// staged in LDS 64 rows at a time as [run][row][R], the order of the output,
+// and leaves in 16-byte vectors, neighbouring lanes on neighbouring addresses.
+template< int MA, int MB >
+__global__ __launch_bounds__( 512, 8 )
+void contract_f32_dma_short_kernel( ContractArgs a ) {
+  constexpr int BM = 128, BN = 128, BK = 32, W = 8, T = 512;
+  typedef F32DmaLoader< BM, BK, W, MA > LdA;
+  typedef F32DmaLoader< BN, BK, W, MB > LdB;
+  constexpr int SA = LdA::STAGE_BYTES, SB = LdB::STAGE_BYTES;
+  __shared__ __attribute__( ( aligned( 1024 ) ) ) char l_lds[SA + SB];
+  __shared__ int32_t l_tab[2 * ( BM + BN )];
+
+  int32_t const l_nblk = gridDim.x;
+  int32_t l_bid = blockIdx.x;
+  if( ( l_nblk & 7 ) == 0 ) l_bid = ( l_bid & 7 ) * ( l_nblk >> 3 ) + ( l_bid >> 3 );
+  int32_t l_c, l_m0, l_n0;
+  decode_tile< BM, BN >( a, l_bid, l_c, l_m0, l_n0 );
+  if( a.out_run > 0 ) l_n0 = l_n0 / BN * a.n_step;
+
+  int const l_lane = threadIdx.x & 63;
+  int const l_wave = __builtin_amdgcn_readfirstlane( threadIdx.x >> 6 );
+  int const l_wm   = l_wave >> 1;
+  int const l_wn   = l_wave & 1;
+
+  i32x4 const l_ra = make_rsrc( reinterpret_cast< float const * >( a.a ) + a.tc_a[l_c], kDmaOob );
+  i32x4 const l_rb = make_rsrc( reinterpret_cast< float const * >( a.b ) + a.tc_b[l_c], kDmaOob );
+  EpilogueTabs< BM, BN, T > l_tabs;
+  {
+    LdA l_lda;
+    LdB l_ldb;
+    l_lda.init( a.tm_a, a.M, l_m0, a.sk_a, l_wave, l_lane );
+    l_ldb.init( a.tn_b, a.N, l_n0, a.sk_b, l_wave, l_lane );
+    uint32_t const l_lds0 = lds_addr( l_lds );
+    static_for< LdA::NJ >( [&]( auto jc ) __attribute__( ( always_inline ) ) {
+      l_lda.template issue_one< decltype( jc )::value >( l_ra, l_lds0, l_wave, 0, a.K, 0u );
+    } );
+    static_for< LdB::NJ >( [&]( auto jc ) __attribute__( ( always_inline ) ) {
+      l_ldb.template issue_one< decltype( jc )::value >( l_rb, l_lds0 + SA, l_wave, 0, a.K, 0u );
+    } );
+  }
+  l_tabs.load( a, l_m0, l_n0 );
+  l_tabs.stage( l_tab );
+
+  F32DmaFrag< BM, BK, 1, MA > l_fra;
+  F32DmaFrag< BN, BK, 2, MB > l_frb;
+  l_fra.init( l_wm * 32, l_lane );
+  l_frb.init( l_wn * 64, l_lane );
+  f32x16 l_acc[1][2] = { { f32x16( 0.0f ), f32x16( 0.0f ) } };
+  wait_vmcnt< 0 >();
+  wait_lgkmcnt0();
+  __syncthreads();
+  static_for< BK / 8 >( [&]( auto sc ) __attribute__( ( always_inline ) ) {
+    constexpr int l_s = decltype( sc )::value;
+    if( l_s > 0 && l_s * 8 >= a.K ) return;
+    f32x4 const l_fa = l_fra.read( l_lds, 0, l_s );
+    f32x4 const l_fb[2] = { l_frb.read( l_lds + SA, 0, l_s ), l_frb.read( l_lds + SA, 1, l_s ) };
+    static_for< 8 >( [&]( auto fc ) __attribute__( ( always_inline ) ) {
+      constexpr int l_f = decltype( fc )::value;
+      l_acc[0][l_f & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32( l_fa[l_f >> 1], l_fb[l_f & 1][l_f >> 1],
+                                                                l_acc[0][l_f & 1], 0, 0, 0 );
+    } );
+  } );
+
+  float * l_base = reinterpret_cast< float * >( a.out ) + a.tc_out[l_c];
+  int32_t const * l_s_m_out = l_tab;
+  int32_t const * l_s_n_out = l_tab + 2 * BM;
+  bool const l_relu = a.last_touch == ETIR_KTYPE_RELU;
+  if( a.out_run == 0 ) {
+    int const l_rows = int( min( int32_t( BM ), a.M - l_m0 ) );
+    int const l_cols = int( min( int32_t( BN ), a.N - l_n0 ) );
+    auto store = [&]( auto relu_c, auto nt_c ) __attribute__( ( always_inline ) ) {
+      constexpr bool RELU = decltype( relu_c )::value, NT = decltype( nt_c )::value;
+      if( l_rows == BM && l_cols == BN ) {
+        epilogue_fast_f32< 1, 2, RELU, false, NT >( l_base, l_acc, l_s_m_out, l_s_n_out, l_wm * 32, l_wn * 64, l_lane );
+      }
+      else {
+        epilogue_fast_f32< 1, 2, RELU, true, NT >( l_base, l_acc, l_s_m_out, l_s_n_out, l_wm * 32, l_wn * 64, l_lane,
+                                                   l_rows, l_cols );
+      }
+    };
+    auto store_nt = [&]( auto relu_c ) __attribute__( ( always_inline ) ) {
+      if( a.out_nt ) store( relu_c, std::true_type() );
+      else           store( relu_c, std::false_type() );
+    };
+    if( l_relu ) store_nt( std::true_type() );
+    else         store_nt( std::false_type() );
+    return;
+  }
+  float * l_tile = reinterpret_cast< float * >( l_lds );
+  constexpr uint32_t HM = BM / 2;                       // rows staged at a time
+  uint32_t const l_R  = uint32_t( a.out_run );
+  uint32_t const l_q  = l_R / 4;                        // vectors per run and row
+  // x / d = umulhi( x, floor( 2^32 / d ) + 1 ), exact for x d < 2^32
+  uint32_t const l_mr = uint32_t( 0xffffffffu / l_R ) + 1u;
+  uint32_t const l_mq = uint32_t( 0xffffffffu / l_q ) + 1u;
+  uint32_t const l_nv = uint32_t( a.n_step ) * ( HM / 4 );
+  int const l_lg = l_lane >> 5;
+#pragma unroll
+  for( int l_h = 0; l_h < 2; l_h++ ) {
+    __syncthreads();                                    // the operands, or the first half, have been read
+    if( ( l_wm >> 1 ) == l_h ) {
+#pragma unroll
+      for( int l_j = 0; l_j < 2; l_j++ ) {
+        uint32_t const l_col = uint32_t( l_wn * 64 + l_j * 32 + ( l_lane & 31 ) );
+        uint32_t const l_run = __umulhi( l_col, l_mr );
+        if( int32_t( l_col ) < a.n_step ) {
+          float * l_p = l_tile + l_run * HM * l_R + ( l_col - l_run * l_R );
+#pragma unroll
+          for( int l_r = 0; l_r < 16; l_r++ ) {
+            float l_v = l_acc[0][l_j][l_r];
+            if( l_relu ) l_v = fmaxf( l_v, 0.0f );
+            l_p[uint32_t( ( l_wm & 1 ) * 32 + 8 * ( l_r >> 2 ) + 4 * l_lg + ( l_r & 3 ) ) * l_R] = l_v;
+          }
+        }
+      }
+    }
+    __syncthreads();
+    for( uint32_t l_e = threadIdx.x; l_e < l_nv; l_e += T ) {
+      uint32_t const l_rr  = __umulhi( l_e, l_mq );     // run * HM + row
+      uint32_t const l_v   = l_e - l_rr * l_q;
+      uint32_t const l_row = l_h * HM + l_rr % HM;
+      uint32_t const l_col = l_rr / HM * l_R;
+      if( l_m0 + int32_t( l_row ) < a.M && l_n0 + int32_t( l_col ) < a.N ) {
+        f32x4 const l_x = *reinterpret_cast< f32x4 const * >( l_tile + 4 * l_e );
+        __builtin_nontemporal_store( l_x, reinterpret_cast< f32x4 * >( l_base + l_s_m_out[l_row] + l_s_n_out[l_col]
+                                                                       + 4 * l_v ) );
+      }
+    }
+  }
+}
+
 }  // namespace kern
 
 int launch_contract_f32_dma( int32_t ma, int32_t mb, ContractArgs const & a, uint32_t grid, hipStream_t stream ) {
@@ -382,7 +523,11 @@ int launch_contract_f32_dma( int32_t ma, int32_t mb, ContractArgs const & a, uin
     return fail( ETIR_COMPILATION_FAILED, "fp32 direct-to-LDS kernel: K table longer than its LDS copy" );
   }
   auto l_go = [&]( auto ma_c, auto mb_c ) {
-    if( a.k_affine ) {
+    if( a.k_one_step ) {
+      hipLaunchKernelGGL( ( kern::contract_f32_dma_short_kernel< decltype( ma_c )::value, decltype( mb_c )::value > ),
+                          dim3( grid ), dim3( 512 ), 0, stream, a );
+    }
+    else if( a.k_affine ) {
       hipLaunchKernelGGL( ( kern::contract_f32_dma_kernel< 128, 128, 32, 4, 2, decltype( ma_c )::value,
                                                            decltype( mb_c )::value, true > ),
                           dim3( grid ), dim3( 512 ), 0, stream, a );

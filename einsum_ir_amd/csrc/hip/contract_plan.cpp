@@ -493,6 +493,8 @@ int plan_contraction_impl( int64_t            num_loops,
       && l_kern_m % 256 == 0 && l_kern_n % 256 == 0 && l_run_n >= 32
       && ( l_run_n % 32 == 0 || l_run_n == l_tn_out.size() )
       && 4 * ( max_of( l_tm_out ) + max_of( l_tn_out ) ) + 4 < ( int64_t( 1 ) << 32 );
+  plan.scattered = l_run_n < 32 && l_run_n < l_tn_out.size() && l_tm_out.size() > 1
+                && l_tm_out[1] != l_tm_out[0] + int64_t( l_run_n );
   if( l_dma_ok && l_persistent && n_tiles( TILE_BF16_DMA_256x256 ) >= l_cus ) plan.tile = TILE_BF16_DMA_256x256;
   else if( l_dma_ok && n_tiles( TILE_BF16_DMA_128x128 ) >= l_cus ) plan.tile = TILE_BF16_DMA_128x128;
   // the fp32 direct-to-LDS kernel: where the planner chose the 128 x 128 fp32
@@ -1079,6 +1081,28 @@ int plan_contraction_impl( int64_t            num_loops,
     a.out_nt = ( l_run >= 32 && ( l_run % 32 == 0 || l_run == l_tn_out.size() ) ) ? 1 : 0;
     if( char const * l_env = std::getenv( "ETIR_OUT_NT" ) ) a.out_nt = std::atoi( l_env ) != 0 ? 1 : 0;
   }
+  // K of one step with plain output: the one-step form of the fp32
+  // direct-to-LDS kernel; there, short output runs whose rows are neighbours
+  // in the output leave by whole runs.  Otherwise for rows of whole 128-byte
+  // lines (20000 x 512 x 32: 14.9 -> 13.4 us; rows of 4100 columns, whose
+  // streamed lines are cut in two, 27.1 -> 28.4 us)
+  bool const l_one_step = plan.tile == TILE_F32_DMA_128x128 && l_k_affine && l_size_k <= 32 && a.out_off32
+                       && ktype_first_touch == ETIR_KTYPE_ZERO
+                       && ( ktype_last_touch == ETIR_KTYPE_UNDEFINED || ktype_last_touch == ETIR_KTYPE_RELU );
+  bool const l_by_runs = l_one_step && l_run_n >= 8 && l_run_n < 32 && l_run_n % 4 == 0
+                      && runs_contiguous( l_tn_out, (int64_t) l_run_n, 4 ) && all_multiple( l_tm_out, 4 )
+                      && all_multiple( l_tc_out, 4 ) && l_tm_out.size() > 1
+                      && l_tm_out[1] == l_tm_out[0] + (int64_t) l_run_n;
+  a.k_one_step = ( l_by_runs || ( l_one_step && all_multiple( l_tm_out, 32 ) && all_multiple( l_tc_out, 32 ) ) ) ? 1 : 0;
+  if( a.k_one_step ) plan.desc += " one_step";
+  a.out_run = 0;
+  a.n_step = 0;
+  if( l_by_runs ) {
+    a.out_run = int32_t( l_run_n );
+    a.n_step  = int32_t( 128 / l_run_n * l_run_n );
+    a.tiles_n = (int32_t) ( ( l_kern_n + a.n_step - 1 ) / a.n_step );
+    plan.desc += " runs=" + std::to_string( l_run_n );
+  }
   if( plan.tile == TILE_PANEL ) {
     int64_t l_mo = 0, l_no = 0;
     for( int64_t l_v : l_tm_out ) l_mo = std::max( l_mo, l_v );
@@ -1119,15 +1143,17 @@ double plan_rate( ContractionPlan const & plan, bool far ) {
 }
 
 // estimated time (us): flops at plan_rate over the useful part of the tile
-// grid, or the tensors' bytes at 3.5 TB/s where that is longer
-double plan_us( ContractionPlan const & plan, bool far, double flops, double bytes ) {
+// grid, or the tensors' bytes at 3.5 TB/s (a scattered output at 2) where that
+// is longer
+double plan_us( ContractionPlan const & plan, bool far, double flops, double bytes_in, double bytes_out ) {
   int64_t l_bm, l_bn;
   tile_shape( plan.tile, l_bm, l_bn );
   double const l_tm = double( ( plan.M + l_bm - 1 ) / l_bm ), l_tn = double( ( plan.N + l_bn - 1 ) / l_bn );
   double const l_tiles = l_tm * l_tn * double( plan.C ) * double( plan.split );
   double const l_util = double( plan.M ) * double( plan.N ) / ( l_tm * double( l_bm ) * l_tn * double( l_bn ) )
                       * std::min( 1.0, l_tiles / 256.0 );
-  return std::max( flops / ( plan_rate( plan, far ) * l_util * 1e6 ), bytes / 3.5e6 ) + 5.0;
+  return std::max( flops / ( plan_rate( plan, far ) * l_util * 1e6 ),
+                   bytes_in / 3.5e6 + bytes_out / ( plan.scattered ? 2.0e6 : 3.5e6 ) ) + 5.0;
 }
 
 // Weighs copying one or both operands K-contiguous into a workspace
@@ -1169,10 +1195,16 @@ void try_pack( int64_t            num_loops,
                bool               allow_split,
                ContractionPlan  & plan ) {
   if( ktype_main != ETIR_KTYPE_MADD || std::getenv( "ETIR_TILE" ) != nullptr ) return;
+  // a side of up to 32 reads the other operand once or twice: a copy of it
+  // reads it as often (efbadx,cfx->abcdex, N = 24: 23.2 ms in place, 25.0 packed)
+  if( std::min( plan.M, plan.N ) <= 32 ) return;
   if( plan.C <= 0 || plan.M <= 0 || plan.N <= 0 || plan.K <= 1 || plan_rate( plan, false ) == 0.0 ) return;
   auto in_vec = [&]( int32_t m ) { return m == LOAD_VEC_MN || m == LOAD_VEC_K; };
   bool const l_affine = ( plan.partial ? plan.partial->args.k_affine : plan.args.k_affine ) != 0;
-  if( in_vec( plan.mode_a ) && in_vec( plan.mode_b ) && ( l_affine || dtype_left == ETIR_FP64 ) ) return;
+  if(    in_vec( plan.mode_a ) && in_vec( plan.mode_b ) && ( l_affine || dtype_left == ETIR_FP64 )
+      && !plan.scattered ) {
+    return;
+  }
 
   int64_t const   l_esz  = dtype_bytes( dtype_left );
   int64_t const   l_vk   = 16 / l_esz;
@@ -1218,8 +1250,8 @@ void try_pack( int64_t            num_loops,
     for( Dim const & l_d : l_rows[l_op] ) l_near = l_near || ( l_d.s == 1 && dim_types[l_d.id] != ETIR_DIM_C );
     l_far = l_far || ( !l_near && l_bytes[l_op] > 4.0e6 );
   }
-  double const l_plain_us = plan_us( plan, l_far, l_flops, l_bytes[0] + l_bytes[1] + l_out );
-  double const l_limit_us = 0.85 * l_plain_us - 2.0;
+  double const l_plain_us = plan_us( plan, l_far, l_flops, l_bytes[0] + l_bytes[1], l_out );
+  double const l_limit_us = 0.93 * l_plain_us - 8.0;
   // not worth planning the alternatives: the fastest kernel and one copy
   double const l_top = dtype_left == ETIR_BF16 ? 1100.0 : ( dtype_left == ETIR_FP64 ? 50.0 : 135.0 );
   double const l_small = std::min( l_bytes[0], l_bytes[1] );
@@ -1288,7 +1320,7 @@ void try_pack( int64_t            num_loops,
     if( plan_rate( l_try, false ) == 0.0 || !in_vec( l_try.mode_a ) || !in_vec( l_try.mode_b ) ) continue;
     // the copies: 8 us each (launch, and the gap before the kernel that reads
     // it) and 2.5 TB/s, read and written
-    l_c.us = plan_us( l_try, false, l_flops, l_bytes[0] + l_bytes[1] + l_out ) + 8.0 * ( l_both ? 2.0 : 1.0 )
+    l_c.us = plan_us( l_try, false, l_flops, l_bytes[0] + l_bytes[1], l_out ) + 8.0 * ( l_both ? 2.0 : 1.0 )
            + 2.0 * l_pack_bytes / 2.5e6;
     // at most 2 GiB of workspace
     if( l_pack_bytes > double( int64_t( 1 ) << 31 ) ) continue;
@@ -1352,6 +1384,8 @@ void try_pack( int64_t            num_loops,
   plan.desc += std::string( " | packed" ) + ( l_best.use[0] ? " left" : "" ) + ( l_best.use[1] ? " right" : "" )
              + ": " + tile_str( l_in.tile ) + " K=" + std::to_string( l_best.pitch ) + " "
              + mode_str( l_in.mode_a ) + " " + mode_str( l_in.mode_b )
+             + ( l_in.args.k_one_step ? " one_step" : "" )
+             + ( l_in.args.out_run > 0 ? " runs=" + std::to_string( l_in.args.out_run ) : std::string() )
              + ( l_pk->cont.split > 1 ? " S=" + std::to_string( l_pk->cont.split ) : std::string() );
 }
 
@@ -1495,7 +1529,13 @@ int launch_contraction( ContractionPlan const & plan,
   a.aux = plan.needs_aux ? out_aux : nullptr;
   a.out = out;
 
-  if( uintptr_t( out ) % 16 != 0 ) a.out_v8 = 0;
+  if( uintptr_t( out ) % 16 != 0 ) {
+    a.out_v8 = 0;
+    if( a.out_run > 0 ) {
+      a.out_run = 0;
+      a.tiles_n = (int32_t) ( ( plan.N + 127 ) / 128 );
+    }
+  }
   // vector paths need aligned base pointers; otherwise fall back to gathers
   int32_t l_ma = plan.mode_a;
   int32_t l_mb = plan.mode_b;

@@ -271,6 +271,10 @@ struct ContractArgs {
   int32_t last_touch;     // ETIR_KTYPE_{RELU,ADD,UNDEFINED}
   int32_t k_full;         // K % BK == 0: no K masking needed
   int32_t out_bf16;       // output stored as bf16 (RNE)
+  int32_t k_one_step;     // fp32 direct-to-LDS kernel: its one-step form (affine K up to 32, plain output)
+  int32_t out_run;        // k_one_step: columns per unit-stride output run (8 to 28, a multiple of 4), the
+                          // output written in 16-byte vectors by runs; 0: column by column
+  int32_t n_step;         // out_run > 0: columns per tile, whole runs
   int32_t out_v8;         // bf16 output in aligned groups of 8 unit-stride columns: 16-byte stores
   int32_t out_off32;      // every output byte offset (M part + N part, C part excluded) is < 2^32
   int32_t c_inner;        // workgroup ids walk C fastest (the output's unit-stride dim is a C dim)
@@ -317,6 +321,8 @@ struct ContractionPlan {
   int32_t mode_b = LOAD_SCALAR;
   int32_t tile = TILE_F32_128x128;
   int32_t tile_fallback = TILE_BF16_256x128;  // used when the DMA kernel's alignment needs fail at launch
+  bool    scattered = false;                  // output rows of under 32 columns whose neighbouring tile rows are not neighbours
+                                              // in the output: lines completed by far-apart stores
   int32_t kwave_waves = 0;                    // TILE_F32_KWAVE_32x32: waves per workgroup and k per wave
   int32_t kwave_kw = 0;
   int32_t dma_variant = 0;                    // 0: BK 64, 2 stages; 1: BK 32, 4 stages, scheduled (VEC_MN x VEC_MN);

@@ -45,7 +45,7 @@ def _error(ref, got):
     ("km,kn->mn", dict(m=1021, n=767, k=769)),
     ("km,nk->nm", dict(m=767, n=1023, k=1025)),                     # roles swapped, one past a vector
     ("zakm,zbkn->zabmn", dict(z=3, a=31, m=21, b=23, n=37, k=517)),  # batch, split rows
-    ("kzml,nlzk->zmn", dict(z=2, m=901, n=703, k=27, l=19)),        # two K dims, opposite orders
+    ("kzml,nlzk->zmn", dict(z=2, m=901, n=703, k=37, l=29)),        # two K dims, opposite orders
     ("aecf,bfde->abcd", dict(a=50, b=50, c=26, d=26, e=24, f=28)),  # K orders conflict
 ])
 def test_packed(torch_cuda, expr, sizes, dtype):

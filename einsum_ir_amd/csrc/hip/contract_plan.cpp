@@ -45,6 +45,7 @@ int launch_contract_panel( ContractArgs const & a, hipStream_t stream );
 int launch_contract_kwave( int32_t waves, int32_t kw, ContractArgs const & a, uint32_t grid,
                            hipStream_t stream );
 int launch_contract_f32_dma( int32_t ma, int32_t mb, ContractArgs const & a, uint32_t grid, hipStream_t stream );
+int launch_contract_f64_dma( ContractArgs const & a, uint32_t grid, hipStream_t stream );
 int launch_contract_gemv( bool bf16_in, ContractArgs const & a, hipStream_t stream );
 int launch_contract_skinny( bool bf16_in, ContractArgs const & a, hipStream_t stream );
 
@@ -158,6 +159,7 @@ char const * tile_str( int32_t t ) {
     case TILE_BF16_128x128: return "bf16_128x128x64";
     case TILE_BF16_64x64:   return "bf16_64x64x64";
     case TILE_F64_64x64:    return "f64_64x64x16";
+    case TILE_F64_DMA_128x128: return "f64_dma_128x128x16";
     case TILE_CPX_F32_64x64: return "cpx_f32_64x64x16";
     case TILE_CPX_F64_64x64: return "cpx_f64_64x64x16";
     case TILE_F32_KWAVE_32x32: return "f32_kwave_32x32";
@@ -181,6 +183,7 @@ void tile_shape( int32_t t, int64_t & bm, int64_t & bn ) {
     case TILE_BF16_128x128: bm = 128; bn = 128; break;
     case TILE_F32_DMA_128x128: bm = 128; bn = 128; break;
     case TILE_BF16_DMA_128x128: bm = 128; bn = 128; break;
+    case TILE_F64_DMA_128x128: bm = 128; bn = 128; break;
     default:                bm = 64;  bn = 64;  break;
   }
 }
@@ -478,6 +481,14 @@ int plan_contraction_impl( int64_t            num_loops,
       && 2 * ( max_of( l_tn_b ) + std::max< int64_t >( l_size_k - 1, 0 ) * l_sk_b ) + 64 < ( int64_t( 1 ) << 31 )
       && 2 * int64_t( 64 ) * std::max( l_sk_a, l_sk_b ) * ( ( l_size_k + 63 ) / 64 + 4 ) < ( int64_t( 1 ) << 31 );
   plan.tile_fallback = plan.tile;
+  // fp64 direct-to-LDS kernel: both operands K-contiguous, byte offsets below
+  // the buffer range (the loads of the step past the last one are issued
+  // too), and the 128 x 128 tiles fill the chip as well as the 64 x 64 ones
+  if(    l_f64 && !l_cpx && plan.mode_a == LOAD_VEC_K && plan.mode_b == LOAD_VEC_K && l_k_affine && l_sk_a == 1
+      && l_sk_b == 1 && 8 * ( std::max( max_of( l_tm_a ), max_of( l_tn_b ) ) + l_size_k + 64 ) < ( int64_t( 1 ) << 31 )
+      && score( TILE_F64_DMA_128x128 ) >= 0.9 * score( TILE_F64_64x64 ) ) {
+    plan.tile = TILE_F64_DMA_128x128;
+  }
   // 256 x 256 tiles where their persistent scheduled loop runs (both operands
   // row-contiguous, whole tiles, plain fp32 output in 32-column runs: 4096 a
   // side 109 us); everything else with a 128 x 128 tile per CU takes those,
@@ -1137,7 +1148,8 @@ double plan_rate( ContractionPlan const & plan, bool far ) {
     case TILE_BF16_256x128:     return by_mode( 550.0, 100.0, 95.0, 20.0 );
     case TILE_BF16_128x128:     return by_mode( 550.0, 50.0, 45.0, 20.0 );
     case TILE_BF16_64x64:       return by_mode( 300.0, 46.0, 45.0, 25.0 );
-    case TILE_F64_64x64:        return by_mode( 50.0, 48.0, 48.0, 18.0 );
+    case TILE_F64_64x64:        return by_mode( plan.args.k_affine ? 50.0 : 43.0, 46.0, 46.0, 18.0 );
+    case TILE_F64_DMA_128x128:  return 64.0;
     default:                    return 0.0;   // not a tile that packing is weighed against
   }
 }
@@ -1201,8 +1213,8 @@ void try_pack( int64_t            num_loops,
   if( plan.C <= 0 || plan.M <= 0 || plan.N <= 0 || plan.K <= 1 || plan_rate( plan, false ) == 0.0 ) return;
   auto in_vec = [&]( int32_t m ) { return m == LOAD_VEC_MN || m == LOAD_VEC_K; };
   bool const l_affine = ( plan.partial ? plan.partial->args.k_affine : plan.args.k_affine ) != 0;
-  if(    in_vec( plan.mode_a ) && in_vec( plan.mode_b ) && ( l_affine || dtype_left == ETIR_FP64 )
-      && !plan.scattered ) {
+  if( in_vec( plan.mode_a ) && in_vec( plan.mode_b ) && l_affine && !plan.scattered
+      && plan.tile != TILE_F64_64x64 ) {
     return;
   }
 
@@ -1253,7 +1265,7 @@ void try_pack( int64_t            num_loops,
   double const l_plain_us = plan_us( plan, l_far, l_flops, l_bytes[0] + l_bytes[1], l_out );
   double const l_limit_us = 0.93 * l_plain_us - 8.0;
   // not worth planning the alternatives: the fastest kernel and one copy
-  double const l_top = dtype_left == ETIR_BF16 ? 1100.0 : ( dtype_left == ETIR_FP64 ? 50.0 : 135.0 );
+  double const l_top = dtype_left == ETIR_BF16 ? 1100.0 : ( dtype_left == ETIR_FP64 ? 64.0 : 135.0 );
   double const l_small = std::min( l_bytes[0], l_bytes[1] );
   if(    std::max( l_flops / ( l_top * 1e6 ), ( l_bytes[0] + l_bytes[1] + l_out ) / 3.5e6 ) + 13.0
        + 2.0 * l_small / 2.5e6 >= l_limit_us ) {
@@ -1550,7 +1562,8 @@ int launch_contraction( ContractionPlan const & plan,
   int32_t l_dma_variant = plan.dma_variant;
   int32_t l_tile = plan.tile;
   if(    ( l_tile == TILE_BF16_DMA_256x256 || l_tile == TILE_BF16_DMA_256x128 || l_tile == TILE_F32_KWAVE_32x32
-           || l_tile == TILE_F32_DMA_128x128 || l_tile == TILE_BF16_DMA_128x128 )
+           || l_tile == TILE_F32_DMA_128x128 || l_tile == TILE_BF16_DMA_128x128
+           || l_tile == TILE_F64_DMA_128x128 )
       && ( l_ma != plan.mode_a || l_mb != plan.mode_b ) ) {
     // the DMA and K-over-waves kernels need the 16-byte vector modes: use
     // the register-staged kernel with its own tile grid
@@ -1577,6 +1590,7 @@ int launch_contraction( ContractionPlan const & plan,
     case TILE_BF16_64x64:
       l_err = launch_contract_tile( l_tile, l_ma, l_mb, l_kaff, a, l_g, stream );
       break;
+    case TILE_F64_DMA_128x128: l_err = launch_contract_f64_dma( a, l_g, stream ); break;
     case TILE_F64_64x64:    l_err = launch_contract_f64_64x64( l_ma, l_mb, l_kaff, a, l_g, stream ); break;
     case TILE_CPX_F32_64x64: l_err = launch_contract_cpx( false, l_ma, l_mb, l_kaff, a, l_g, stream ); break;
     case TILE_CPX_F64_64x64: l_err = launch_contract_cpx( true, l_ma, l_mb, l_kaff, a, l_g, stream ); break;

@@ -240,6 +240,7 @@ enum TileCfg : int32_t {
   TILE_GEMV             = 13, // M == 1 or N == 1: one thread per output element (contract_gemv.hip)
   TILE_SKINNY           = 14, // one free side of 2-64: one thread per long index (contract_skinny.hip)
   TILE_BF16_DMA_128x128 = 16, // bf16 direct-to-LDS kernel, two workgroups per CU, any pairing of the vector modes
+  TILE_F64_DMA_128x128  = 17, // fp64 direct-to-LDS kernel, both operands K-contiguous (contract_f64_dma.hip)
   TILE_PANEL            = 15  // short K, one free side of 65-256 resident in LDS (contract_panel.hip)
 };
 

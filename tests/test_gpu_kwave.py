@@ -42,3 +42,11 @@ def test_kwave_matches_split_k(torch_cuda, oracle, monkeypatch):
     got_s, desc_s = run_case(torch_cuda, oracle, "mk,nk->mn", dict(m=256, n=512, k=1024), seed=41)
     assert "kwave" in desc_w and "kwave" not in desc_s, (desc_w, desc_s)
     assert np.linalg.norm(got_w - got_s) / np.linalg.norm(got_s) <= 1e-5
+
+
+@pytest.mark.parametrize("m,n,k", [(64, 64, 96), (128, 100, 112), (33, 47, 240), (256, 256, 256), (1, 33, 304),
+                                   (100, 100, 496), (128, 128, 512)])
+def test_kwave_few_tiles(torch_cuda, oracle, m, n, k):
+    """Few tiles and a K of 96 to 512: waves whose K range is short or empty."""
+    _, desc = run_case(torch_cuda, oracle, "mk,nk->mn", dict(m=m, n=n, k=k), seed=k)
+    assert m == 1 or "f32_kwave_32x32" in desc, desc

@@ -1233,6 +1233,7 @@ void try_pack( int64_t            num_loops,
     int64_t l_n = 1;
     for( int64_t l_lo = 0; l_lo < num_loops; l_lo++ ) {
       if( sizes[l_lo] <= 1 || dim_types[l_lo] == ETIR_DIM_I || dim_types[l_lo] == ETIR_DIM_J ) continue;
+      if( dim_types[l_lo] == ( l_op == 0 ? ETIR_DIM_N : ETIR_DIM_M ) ) continue;
       bool const l_is_k = dim_types[l_lo] == ETIR_DIM_K;
       if( l_st[l_op][l_lo] == 0 ) {
         if( l_is_k ) return;                // a K loop that an operand does not move along

@@ -1390,7 +1390,12 @@ void try_pack( int64_t            num_loops,
                                 dtype_comp, dtype_out, ktype_first_touch, ktype_main, ktype_last_touch, allow_split,
                                 l_pk->cont, nullptr ) != ETIR_SUCCESS
       || hipMalloc( &l_pk->ws, (std::size_t) l_total ) != hipSuccess
-      || ( l_best.pitch != plan.K && hipMemset( l_pk->ws, 0, (std::size_t) l_total ) != hipSuccess )
+      // the padding's zeros are there when this returns: the fill runs on the
+      // null stream, which a non-blocking stream's first execution does not
+      // wait for, and hipMemset may return before it has run
+      || (    l_best.pitch != plan.K
+           && (    hipMemset( l_pk->ws, 0, (std::size_t) l_total ) != hipSuccess
+                || hipStreamSynchronize( nullptr ) != hipSuccess ) )
       || hipEventCreateWithFlags( &l_pk->done, hipEventDisableTiming ) != hipSuccess ) {
     drop();
     return;

@@ -6,6 +6,8 @@ kernels, several streams, and stream capture (which reads them in place).
 Checker: torch.einsum in 64 bits on the same values.  Bars: fp32 1e-5 and
 bf16 2e-3 relative Frobenius (fp32 sums of exact products), fp64 1e-12.
 """
+import ctypes
+
 import pytest
 
 import einsum_ir_amd as eir
@@ -106,6 +108,35 @@ def test_packed_on_several_streams(torch_cuda):
     for (a, b, _), out in zip(sets, outs):
         assert _error(torch.einsum(expr, a.double(), b.double()), out) <= TOL_FP32
     plan.close()
+
+
+def test_packed_padding_is_cleared_before_the_first_execution(torch_cuda):
+    """Rows padded from 1019 to 1020: the first execution, on a stream that does
+    not wait for the null stream, follows the plan's creation with nothing
+    waited for in between, in memory that held NaN before."""
+    torch = torch_cuda
+    expr, sizes = "mk,nk->mn", dict(m=1023, n=1021, k=1019)
+    lib = eir.hip_lib()
+    a, b, shape = _operands(torch, expr, sizes, "float32", 40)
+    ref = torch.einsum(expr, a.double(), b.double())
+    outs = [torch.full(shape, float("nan"), device="cuda") for _ in range(4)]
+    stream = ctypes.c_void_p()
+    eir.check(lib.etir_hip_stream_create(ctypes.byref(stream)))
+    for out in outs:
+        # the workspace is likely to be this block again
+        block = ctypes.c_void_p()
+        eir.check(lib.etir_hip_malloc(ctypes.byref(block), 4 * 1020 * (1023 + 1021)))
+        eir.check(lib.etir_hip_memset(block, 0xff, 4 * 1020 * (1023 + 1021)))
+        torch.cuda.synchronize()
+        eir.check(lib.etir_hip_free(block))
+        plan = _plan(expr, sizes, "float32")
+        plan.execute(a, b, out, stream=stream.value)
+        assert "packed" in plan.describe(), plan.describe()
+        eir.synchronize(stream.value)
+        plan.close()
+    eir.check(lib.etir_hip_stream_destroy(stream))
+    for out in outs:
+        assert _error(ref, out) <= TOL_FP32
 
 
 def test_packed_plan_under_capture(torch_cuda):

@@ -1459,9 +1459,10 @@ void release_contraction( ContractionPlan & plan ) {
 }
 
 // The packed form of a contraction on `stream`.  The workspace is the plan's
-// one: an execution on another stream than the last waits for that one's end
-// (also on the per-thread default stream, whose one handle names a stream per
-// thread).
+// one: every execution waits for the end of the last one.  Also on the same
+// stream handle, where the wait costs nothing: a handle names another stream
+// once the first has been destroyed (its work may still run) or, for the
+// per-thread default stream, in another thread.
 static int launch_packed( PackedContraction & pk,
                           void const        * left,
                           void const        * right,
@@ -1469,9 +1470,7 @@ static int launch_packed( PackedContraction & pk,
                           void              * out,
                           hipStream_t         stream ) {
   std::lock_guard< std::mutex > l_guard( pk.lock );
-  if( pk.ran && ( pk.stream != stream || stream == hipStreamPerThread ) ) {
-    ETIR_HIP_CHECK( hipStreamWaitEvent( stream, pk.done, 0 ) );
-  }
+  if( pk.ran ) ETIR_HIP_CHECK( hipStreamWaitEvent( stream, pk.done, 0 ) );
   void const * l_op[2] = { left, right };
   int l_err = ETIR_SUCCESS;
   for( int l_i = 0; l_i < 2 && l_err == ETIR_SUCCESS; l_i++ ) {
@@ -1483,7 +1482,6 @@ static int launch_packed( PackedContraction & pk,
   if( l_err == ETIR_SUCCESS ) l_err = launch_contraction( pk.cont, l_op[0], l_op[1], out_aux, out, stream );
   // recorded after an error too: what was enqueued still uses the workspace
   pk.ran = true;
-  pk.stream = stream;
   ETIR_HIP_CHECK( hipEventRecord( pk.done, stream ) );
   return l_err;
 }

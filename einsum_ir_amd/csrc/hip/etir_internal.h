@@ -360,8 +360,8 @@ struct ContractionPlan {
 
 // A contraction over K-contiguous copies of one or both operands (slots: 0
 // left, 1 right): two permutations into the plan's workspace, then `cont` on
-// them.  One workspace for all executions: an execution on another stream
-// than the last one waits for `done`, which every execution records.
+// them.  One workspace for all executions: each waits for `done`, which the
+// one before recorded.
 struct PackedContraction {
   ContractionPlan cont;
   PermutePlan perm[2];
@@ -370,7 +370,6 @@ struct PackedContraction {
   int64_t     offset[2] = { 0, 0 };     // bytes into ws
   std::mutex  lock;
   hipEvent_t  done   = nullptr;
-  hipStream_t stream = nullptr;         // of the last execution
   bool        ran    = false;
 };
 

@@ -139,6 +139,28 @@ def test_packed_padding_is_cleared_before_the_first_execution(torch_cuda):
         assert _error(ref, out) <= TOL_FP32
 
 
+def test_packed_on_a_recycled_stream(torch_cuda):
+    """A stream destroyed with an execution in flight; the next one may get its
+    handle and still waits for that execution."""
+    torch = torch_cuda
+    expr, sizes = "mk,nk->mn", dict(m=2047, n=2045, k=2043)
+    lib = eir.hip_lib()
+    plan = _plan(expr, sizes, "float32")
+    assert "packed" in plan.describe(), plan.describe()
+    sets = [_operands(torch, expr, sizes, "float32", 50 + i) for i in range(4)]
+    outs = [torch.full(s[2], float("nan"), device="cuda") for s in sets]
+    torch.cuda.synchronize()
+    for (a, b, _), out in zip(sets, outs):
+        stream = ctypes.c_void_p()
+        eir.check(lib.etir_hip_stream_create(ctypes.byref(stream)))
+        plan.execute(a, b, out, stream=stream.value)
+        eir.check(lib.etir_hip_stream_destroy(stream))
+    torch.cuda.synchronize()
+    for (a, b, _), out in zip(sets, outs):
+        assert _error(torch.einsum(expr, a.double(), b.double()), out) <= TOL_FP32
+    plan.close()
+
+
 def test_packed_plan_under_capture(torch_cuda):
     """A captured execution reads its operands in place: replays, with eager
     executions of the same plan on another stream between them, stay right."""

@@ -26,6 +26,7 @@
 //   5. the tile shape is chosen from dtype and the number of output tiles.
 #include "etir_internal.h"
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <limits>
@@ -223,7 +224,8 @@ int plan_contraction_impl( int64_t            num_loops,
                            ContractionPlan  & plan,
                            DevicePlacement  * place,
                            bool               dry = false ) {
-  // dry: tile, load modes and split only, no device memory
+  // dry: tile, load modes and split (those of its partial contraction) only,
+  // no device memory
   plan = ContractionPlan();
   plan.placed = ( place != nullptr );
 
@@ -701,25 +703,46 @@ int plan_contraction_impl( int64_t            num_loops,
       std::vector< Loop > l_kk = l_k;          // K loops, outer -> inner
       std::vector< Loop > l_sp;                // split parts, outer -> inner
       int64_t l_sf = 1;
+      bool const l_vec_k = plan.mode_a != LOAD_SCALAR && plan.mode_b != LOAD_SCALAR
+                        && ( plan.mode_a == LOAD_VEC_K || plan.mode_b == LOAD_VEC_K );
       std::size_t l_i = 0;
       while( l_sf < l_target && l_i < l_kk.size() ) {
         Loop & l_lp = l_kk[l_i];
         int64_t const l_need = ( l_target + l_sf - 1 ) / l_sf;
         // factor of this loop: the smallest divisor that reaches the target,
         // else the largest one that stays within l_smax
-        // (first pass: where this is the innermost K loop and unit-stride in
-        // an operand, only factors that leave its inner part a multiple of 4,
-        // so that K rows stay 16-byte loadable: 4620 = 4 x 1155 on the fp32
-        // direct-to-LDS kernel measured 457 us, 5 x 924 the vector loads)
+        // (first pass: only factors that leave the K of a split a multiple of
+        // l_q, so that its rows stay loadable in vectors: 4620 = 4 x 1155 on
+        // the fp32 direct-to-LDS kernel measured 457 us, 5 x 924 the vector
+        // loads; bf16 2384 = 4 x 596 gathers element by element, 2 x 1192 not;
+        // fp32 loops that run on in memory 8-byte vectors at least: 136 x 792
+        // x (54 x 18) 11.9 us in 6 x 162, 14.2 in 3 x 324)
+        int64_t l_in = 1;                        // K of the loops inside this one
+        for( std::size_t l_j = l_i + 1; l_j < l_kk.size(); l_j++ ) l_in *= l_kk[l_j].size;
+        int64_t l_q = 1;
+        if( l_in == 1 && l_lp.size % 4 == 0 && ( l_lp.s[T_L] == 1 || l_lp.s[T_R] == 1 ) ) l_q = 4;
+        if( l_vec_k ) l_q = std::max( l_q, l_f32 ? int64_t( 2 ) : l_vk );
         int64_t l_f = 0;
-        bool const l_keep4 = l_i + 1 == l_kk.size() && l_lp.size % 4 == 0
-                          && ( l_lp.s[T_L] == 1 || l_lp.s[T_R] == 1 );
-        for( int l_pass = l_keep4 ? 0 : 1; l_pass < 2 && l_f == 0; l_pass++ ) {
+        for( int l_pass = l_q > 1 ? 0 : 1; l_pass < 2 && l_f == 0; l_pass++ ) {
           for( int64_t l_d = 2; l_d <= l_lp.size; l_d++ ) {
             if( l_lp.size % l_d != 0 || l_sf * l_d > l_smax ) continue;
-            if( l_pass == 0 && ( l_lp.size / l_d ) % 4 != 0 ) continue;
+            if( l_pass == 0 && ( l_lp.size / l_d * l_in ) % l_q != 0 ) continue;
             l_f = l_d;
             if( l_d >= l_need ) break;
+          }
+          // giving up vector loads pays from 8 splits on (bf16: and a K of
+          // 4096), in fp32 also from 4 on where the operands are small (split /
+          // whole, bf16 256 x 256: K = 2056 in 2 80 / 16 us, in 8 20 / 16, 4184
+          // in 8 34 / 42, 16408 in 14 99 / 146; fp32 in 4, 128 x 128: K = 2092
+          // 41 / 50, 4252 77 / 98, 6044 188 / 138; 256 x 256: 2092 44 / 50, 3028
+          // 82 / 71; 512 x 384: 2092 63 / 50)
+          if( l_pass == 1 && l_vec_k ) {
+            int64_t const l_s   = l_sf * l_f;
+            int64_t const l_out = l_size_c * l_size_m * l_size_n;
+            bool const l_pays = l_f32 ? l_s >= 8 || (    l_s >= 4 && l_out <= 65536
+                                                     && l_size_k < ( l_out <= 16384 ? 4608 : 2560 ) )
+                                      : l_s >= 8 && l_size_k >= 4096;
+            if( !l_pays ) l_f = 0;
           }
         }
         if( l_f == 0 ) break;
@@ -793,14 +816,6 @@ int plan_contraction_impl( int64_t            num_loops,
       }
       int64_t const l_ws_bytes = 4 * l_sf * l_span;
       if( l_sf >= 2 && l_size_k / l_sf >= 128 && l_ws_bytes <= ( int64_t( 1 ) << 29 ) ) {
-        if( dry ) {
-          plan.split = (int32_t) l_sf;
-          plan.C = l_size_c;
-          plan.M = l_kern_m;
-          plan.N = l_kern_n;
-          plan.K = l_size_k;
-          return ETIR_SUCCESS;
-        }
         // loop arrays of the partial contraction
         std::vector< int32_t > l_pt;
         std::vector< int64_t > l_psz, l_pl, l_pr, l_pa, l_po;
@@ -824,10 +839,22 @@ int plan_contraction_impl( int64_t            num_loops,
         int l_err = plan_contraction_impl( (int64_t) l_pt.size(), l_pt.data(), l_psz.data(), l_pl.data(),
                                            l_pr.data(), l_pa.data(), l_po.data(), dtype_left, dtype_right,
                                            ETIR_FP32, ETIR_FP32, ETIR_KTYPE_ZERO, ETIR_KTYPE_MADD,
-                                           ETIR_KTYPE_UNDEFINED, false, *l_part, place );
+                                           ETIR_KTYPE_UNDEFINED, false, *l_part, place, dry );
         if( l_err != ETIR_SUCCESS ) {
           release_contraction( *l_part );
           return l_err;
+        }
+        plan.args.k_affine = l_part->args.k_affine;
+        if( dry ) {
+          plan.split  = (int32_t) l_sf;
+          plan.C      = l_size_c;
+          plan.M      = l_part->M;
+          plan.N      = l_part->N;
+          plan.K      = l_size_k;
+          plan.mode_a = l_part->mode_a;
+          plan.mode_b = l_part->mode_b;
+          plan.tile   = l_part->tile;
+          return ETIR_SUCCESS;
         }
         if( place != nullptr ) {
           l_err = place_take( *place, (std::size_t) l_ws_bytes, &plan.d_ws, "split-K workspace" );
@@ -1145,28 +1172,31 @@ double plan_rate( ContractionPlan const & plan, bool far ) {
   switch( plan.tile ) {
     case TILE_F32_DMA_128x128:  return 135.0;
     case TILE_F32_128x128:      return by_mode( 112.0, 75.0, 75.0, 16.0 );
-    case TILE_F32_64x64:        return by_mode( 65.0, 30.0, 25.0, 25.0 );
-    case TILE_BF16_DMA_256x256: return plan.mode_a == LOAD_VEC_MN && plan.mode_b == LOAD_VEC_MN ? 1100.0 : 800.0;
+    case TILE_F32_64x64:        return by_mode( 78.0, plan.args.k_affine && plan.split > 1 ? 36.0 : 30.0, 25.0, 25.0 );
+    case TILE_F32_KWAVE_32x32:  return 50.0;
+    case TILE_BF16_DMA_256x256: return 1100.0;
     case TILE_BF16_DMA_128x128: return 850.0;
     case TILE_BF16_256x128:     return by_mode( 550.0, 100.0, 95.0, 20.0 );
-    case TILE_BF16_128x128:     return by_mode( 550.0, 50.0, 45.0, 20.0 );
+    case TILE_BF16_128x128:     return by_mode( 550.0, plan.args.k_affine ? 80.0 : 50.0, 45.0, 20.0 );
     case TILE_BF16_64x64:       return by_mode( 300.0, 46.0, 45.0, 25.0 );
-    case TILE_F64_64x64:        return by_mode( plan.args.k_affine ? 50.0 : 43.0, 46.0, 46.0, 18.0 );
-    case TILE_F64_DMA_128x128:  return 64.0;
+    case TILE_F64_64x64:        return by_mode( plan.args.k_affine ? 48.0 : 41.0, 46.0, 46.0, 18.0 );
+    case TILE_F64_DMA_128x128:  return 68.0;
     default:                    return 0.0;   // not a tile that packing is weighed against
   }
 }
 
 // estimated time (us): flops at plan_rate over the useful part of the tile
 // grid, or the tensors' bytes at 3.5 TB/s (a scattered output at 2) where that
-// is longer
+// is longer.  fp64 tiles run in whole rounds of one per CU (2100 a side, 289
+// tiles of 128 x 128, takes as long as 2500 with 400)
 double plan_us( ContractionPlan const & plan, bool far, double flops, double bytes_in, double bytes_out ) {
   int64_t l_bm, l_bn;
   tile_shape( plan.tile, l_bm, l_bn );
   double const l_tm = double( ( plan.M + l_bm - 1 ) / l_bm ), l_tn = double( ( plan.N + l_bn - 1 ) / l_bn );
   double const l_tiles = l_tm * l_tn * double( plan.C ) * double( plan.split );
+  bool const l_f64 = plan.tile == TILE_F64_64x64 || plan.tile == TILE_F64_DMA_128x128;
   double const l_util = double( plan.M ) * double( plan.N ) / ( l_tm * double( l_bm ) * l_tn * double( l_bn ) )
-                      * std::min( 1.0, l_tiles / 256.0 );
+                      * ( l_f64 ? l_tiles / ( 256.0 * std::ceil( l_tiles / 256.0 ) ) : std::min( 1.0, l_tiles / 256.0 ) );
   return std::max( flops / ( plan_rate( plan, far ) * l_util * 1e6 ),
                    bytes_in / 3.5e6 + bytes_out / ( plan.scattered ? 2.0e6 : 3.5e6 ) ) + 5.0;
 }
@@ -1215,7 +1245,7 @@ void try_pack( int64_t            num_loops,
   if( std::min( plan.M, plan.N ) <= 32 ) return;
   if( plan.C <= 0 || plan.M <= 0 || plan.N <= 0 || plan.K <= 1 || plan_rate( plan, false ) == 0.0 ) return;
   auto in_vec = [&]( int32_t m ) { return m == LOAD_VEC_MN || m == LOAD_VEC_K; };
-  bool const l_affine = ( plan.partial ? plan.partial->args.k_affine : plan.args.k_affine ) != 0;
+  bool const l_affine = plan.args.k_affine != 0;
   if( in_vec( plan.mode_a ) && in_vec( plan.mode_b ) && l_affine && !plan.scattered
       && plan.tile != TILE_F64_64x64 ) {
     return;
@@ -1269,7 +1299,7 @@ void try_pack( int64_t            num_loops,
   double const l_plain_us = plan_us( plan, l_far, l_flops, l_bytes[0] + l_bytes[1], l_out );
   double const l_limit_us = 0.93 * l_plain_us - 8.0;
   // not worth planning the alternatives: the fastest kernel and one copy
-  double const l_top = dtype_left == ETIR_BF16 ? 1100.0 : ( dtype_left == ETIR_FP64 ? 64.0 : 135.0 );
+  double const l_top = dtype_left == ETIR_BF16 ? 1100.0 : ( dtype_left == ETIR_FP64 ? 68.0 : 135.0 );
   double const l_small = std::min( l_bytes[0], l_bytes[1] );
   if(    std::max( l_flops / ( l_top * 1e6 ), ( l_bytes[0] + l_bytes[1] + l_out ) / 3.5e6 ) + 13.0
        + 2.0 * l_small / 2.5e6 >= l_limit_us ) {
@@ -1283,13 +1313,30 @@ void try_pack( int64_t            num_loops,
   };
   struct Choice { double us; bool use[2]; Loops loops; int order; int64_t pitch; };
   Choice l_best{ l_limit_us, { false, false }, {}, 0, 0 };
+  // row length of the copies where both are made: whole vectors, and where few
+  // tiles and a long K ask for a split, the next length that divides into
+  // enough parts of whole vectors (bf16 ea,ebcd->abcd 256,4562,99: 4568 = 8 x
+  // 571 in 2 parts that gather element by element 179 us)
+  int64_t l_pitch = ( plan.K + l_vk - 1 ) / l_vk * l_vk;
+  if( allow_split && dtype_left != ETIR_FP64 && plan.K >= 512 ) {
+    int64_t const l_t = ( plan.M + 63 ) / 64 * ( ( plan.N + 63 ) / 64 ) * plan.C;
+    int64_t const l_parts = l_t < 256 ? std::min( ( 512 + l_t - 1 ) / l_t, plan.K / 128 ) : 1;
+    auto divides = [&]( int64_t k ) {
+      for( int64_t l_d = l_parts; l_d < 2 * l_parts && l_d * 128 <= k; l_d++ ) {
+        if( k % ( l_d * l_vk ) == 0 ) return true;
+      }
+      return false;
+    };
+    // (a multiple of l_parts vectors is at most that many vectors away)
+    while( !divides( l_pitch ) ) l_pitch += l_vk;
+  }
   for( int l_ch = 1; l_ch < 4; l_ch++ ) {
     bool const l_use[2] = { ( l_ch & 1 ) != 0, ( l_ch & 2 ) != 0 };
     bool const l_both = l_use[0] && l_use[1];
     Choice l_c{ 0.0, { l_use[0], l_use[1] }, {}, 0, 0 };
     // K order: that of the operand read in place, or of the larger one
     l_c.order = l_both ? ( l_bytes[0] >= l_bytes[1] ? 0 : 1 ) : ( l_use[0] ? 1 : 0 );
-    l_c.pitch = l_both ? ( plan.K + l_vk - 1 ) / l_vk * l_vk : plan.K;
+    l_c.pitch = l_both ? l_pitch : plan.K;
     Loops & l_lp = l_c.loops;
     double l_pack_bytes = 0.0;
     std::vector< int64_t > l_packed[2];      // stride per loop of a copied operand

@@ -62,6 +62,26 @@ def test_packed(torch_cuda, expr, sizes, dtype):
     plan.close()
 
 
+@pytest.mark.parametrize("expr,sizes,dtype", [
+    ("mk,nk->mn", dict(m=767, n=769, k=773), "bfloat16"),               # 776 = 8 x 97
+    ("mk,nk->mn", dict(m=1021, n=1023, k=1041), "bfloat16"),            # 1048 = 8 x 131
+    ("eafd,fbec->abcd", dict(a=10, d=9, c=75, b=64, f=39, e=61), "bfloat16"),   # 2384 = 16 x 149
+    ("abkl,cdkl->abcd", dict(a=31, b=8, d=13, c=24, k=92, l=61), "float32"),
+])
+def test_packed_kernels_load_vectors(torch_cuda, expr, sizes, dtype):
+    """Where K of the copies is split, the parts keep the vector loads that the
+    copies are made for."""
+    torch = torch_cuda
+    a, b, shape = _operands(torch, expr, sizes, dtype, 17)
+    out = torch.full(shape, float("nan"), device="cuda")
+    plan = _plan(expr, sizes, dtype)
+    desc = plan.describe()
+    assert " | packed" not in desc or "scalar" not in desc.split(" | packed")[1], desc
+    plan.execute(a, b, out, stream=torch.cuda.current_stream())
+    assert _error(torch.einsum(expr, a.double(), b.double()), out) <= TOL[dtype]
+    plan.close()
+
+
 def test_packed_fp64_and_unaligned(torch_cuda):
     """fp64 with conflicting K orders; operands one element off alignment."""
     torch = torch_cuda

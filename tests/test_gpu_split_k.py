@@ -120,3 +120,26 @@ def test_split_matches_unsplit(torch_cuda, oracle, monkeypatch):
     assert _split_of(desc_s) > 1 and _split_of(desc_u) == 1, (desc_s, desc_u)
     err = np.linalg.norm(got_s - got_u) / np.linalg.norm(got_u)
     assert err <= 1e-5
+
+
+@pytest.mark.parametrize("dtype,m,n,k,split,mode", [
+    ("bf16", 256, 256, 2384, 2, "vec_k"),    # 16 x 149: K' = 1192, in 4 it would not be a multiple of 8
+    ("bf16", 256, 256, 2056, 1, "vec_k"),    # 8 x 257: no split keeps 16-byte rows
+    ("bf16", 256, 256, 4184, 8, "scalar"),   # 8 x 523: 8 splits outweigh the vector loads
+    ("bf16", 64, 64, 16408, 7, "vec_k"),     # 8 x 7 x 293
+    ("fp32", 512, 384, 2092, 1, "vec_k"),    # 4 x 523
+    ("fp32", 64, 64, 2092, 4, "scalar"),     # one tile: 4 splits outweigh the vector loads
+    ("fp32", 96, 64, 4620, 35, "vec_k"),     # K' = 132
+])
+def test_split_keeps_vector_loads(torch_cuda, oracle, dtype, m, n, k, split, mode):
+    _, desc = run_case(torch_cuda, oracle, "mk,nk->mn", dict(m=m, n=n, k=k),
+                       dtype=eir.BF16 if dtype == "bf16" else eir.FP32, seed=77)
+    assert _split_of(desc) == split, desc
+    assert "A=left:%s B=right:%s" % (mode, mode) in desc, desc
+
+
+def test_split_of_merged_k_loops_keeps_vector_loads(torch_cuda, oracle):
+    """Two adjacent K dims, 92 x 61: a split of the outer one leaves a multiple
+    of 61, which is one of 4 only where its inner part is."""
+    _, desc = run_case(torch_cuda, oracle, "mkl,nkl->mn", dict(m=300, n=200, k=92, l=61), seed=78)
+    assert "scalar" not in desc, desc

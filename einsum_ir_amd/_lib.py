@@ -40,6 +40,7 @@ _HIP_SIGS = {
                                                    ctypes.c_int32, ctypes.c_int32, ctypes.c_int32,
                                                    ctypes.POINTER(_vp)]),
     "etir_hip_contraction_execute": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _vp]),
+    "etir_hip_contraction_execute_ordered": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _vp]),
     "etir_hip_permute_create": (ctypes.c_int, [ctypes.c_int64, _i64p, _i64p, _i64p, ctypes.c_int32,
                                                ctypes.c_int32, ctypes.c_int32, ctypes.c_int32,
                                                ctypes.POINTER(_vp)]),

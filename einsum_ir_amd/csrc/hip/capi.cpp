@@ -73,7 +73,20 @@ int etir_hip_contraction_execute( etir_plan_t  plan,
     return fail( ETIR_CALLED_BEFORE_COMPILATION, "not a contraction plan" );
   }
   return etir::launch_contraction( plan->cont, left, right, out_aux, out,
-                                   reinterpret_cast< hipStream_t >( stream ) );
+                                   reinterpret_cast< hipStream_t >( stream ), false );
+}
+
+int etir_hip_contraction_execute_ordered( etir_plan_t  plan,
+                                          void const * left,
+                                          void const * right,
+                                          void const * out_aux,
+                                          void       * out,
+                                          void       * stream ) {
+  if( plan == nullptr || plan->kind != 1 ) {
+    return fail( ETIR_CALLED_BEFORE_COMPILATION, "not a contraction plan" );
+  }
+  return etir::launch_contraction( plan->cont, left, right, out_aux, out,
+                                   reinterpret_cast< hipStream_t >( stream ), true );
 }
 
 int etir_hip_permute_create( int64_t         num_dims,

@@ -1396,7 +1396,6 @@ void try_pack( int64_t            num_loops,
     release_contraction( l_pk->cont );
     for( PermutePlan & l_p : l_pk->perm ) release_permute( l_p );
     if( l_pk->ws != nullptr ) (void) hipFree( l_pk->ws );
-    if( l_pk->done != nullptr ) (void) hipEventDestroy( l_pk->done );
     (void) hipGetLastError();
   };
   int64_t l_total = 0;
@@ -1442,8 +1441,7 @@ void try_pack( int64_t            num_loops,
       // wait for, and hipMemset may return before it has run
       || (    l_best.pitch != plan.K
            && (    hipMemset( l_pk->ws, 0, (std::size_t) l_total ) != hipSuccess
-                || hipStreamSynchronize( nullptr ) != hipSuccess ) )
-      || hipEventCreateWithFlags( &l_pk->done, hipEventDisableTiming ) != hipSuccess ) {
+                || hipStreamSynchronize( nullptr ) != hipSuccess ) ) ) {
     drop();
     return;
   }
@@ -1483,6 +1481,10 @@ int plan_contraction( int64_t            num_loops,
   if( l_err == ETIR_SUCCESS && place == nullptr ) {
     try_pack( num_loops, dim_types, sizes, strides_left, strides_right, strides_out_aux, strides_out, dtype_left,
               dtype_right, dtype_comp, dtype_out, ktype_first_touch, ktype_main, ktype_last_touch, l_split, plan );
+    if( plan.packed || plan.split > 1 ) {
+      plan.order = std::make_shared< ExecOrder >();
+      ETIR_HIP_CHECK( hipEventCreateWithFlags( &plan.order->done, hipEventDisableTiming ) );
+    }
   }
   return l_err;
 }
@@ -1500,37 +1502,37 @@ void release_contraction( ContractionPlan & plan ) {
     release_contraction( plan.packed->cont );
     for( PermutePlan & l_p : plan.packed->perm ) release_permute( l_p );
     if( plan.packed->ws != nullptr ) (void) hipFree( plan.packed->ws );
-    if( plan.packed->done != nullptr ) (void) hipEventDestroy( plan.packed->done );
     plan.packed.reset();
+  }
+  if( plan.order ) {
+    if( plan.order->done != nullptr ) (void) hipEventDestroy( plan.order->done );
+    plan.order.reset();
   }
 }
 
-// The packed form of a contraction on `stream`.  The workspace is the plan's
-// one: every execution waits for the end of the last one.  Also on the same
-// stream handle, where the wait costs nothing: a handle names another stream
-// once the first has been destroyed (its work may still run) or, for the
-// per-thread default stream, in another thread.
-static int launch_packed( PackedContraction & pk,
-                          void const        * left,
-                          void const        * right,
-                          void const        * out_aux,
-                          void              * out,
-                          hipStream_t         stream ) {
-  std::lock_guard< std::mutex > l_guard( pk.lock );
-  if( pk.ran ) ETIR_HIP_CHECK( hipStreamWaitEvent( stream, pk.done, 0 ) );
+static int enqueue( ContractionPlan const & plan,
+                    void const            * left,
+                    void const            * right,
+                    void const            * out_aux,
+                    void                  * out,
+                    hipStream_t             stream );
+
+// the packed form of a contraction
+static int enqueue_packed( PackedContraction const & pk,
+                           void const              * left,
+                           void const              * right,
+                           void const              * out_aux,
+                           void                    * out,
+                           hipStream_t               stream ) {
   void const * l_op[2] = { left, right };
-  int l_err = ETIR_SUCCESS;
-  for( int l_i = 0; l_i < 2 && l_err == ETIR_SUCCESS; l_i++ ) {
+  for( int l_i = 0; l_i < 2; l_i++ ) {
     if( !pk.use[l_i] ) continue;
     void * l_copy = static_cast< char * >( pk.ws ) + pk.offset[l_i];
-    l_err = launch_permute( pk.perm[l_i], l_op[l_i], l_copy, stream );
+    int l_err = launch_permute( pk.perm[l_i], l_op[l_i], l_copy, stream );
+    if( l_err != ETIR_SUCCESS ) return l_err;
     l_op[l_i] = l_copy;
   }
-  if( l_err == ETIR_SUCCESS ) l_err = launch_contraction( pk.cont, l_op[0], l_op[1], out_aux, out, stream );
-  // recorded after an error too: what was enqueued still uses the workspace
-  pk.ran = true;
-  ETIR_HIP_CHECK( hipEventRecord( pk.done, stream ) );
-  return l_err;
+  return enqueue( pk.cont, l_op[0], l_op[1], out_aux, out, stream );
 }
 
 int launch_contraction( ContractionPlan const & plan,
@@ -1538,7 +1540,8 @@ int launch_contraction( ContractionPlan const & plan,
                         void const            * right,
                         void const            * out_aux,
                         void                  * out,
-                        hipStream_t             stream ) {
+                        hipStream_t             stream,
+                        bool                    ordered ) {
   if( plan.C == 0 || plan.M == 0 || plan.N == 0 ) return ETIR_SUCCESS;
   if( out == nullptr || ( plan.K > 0 && ( left == nullptr || right == nullptr ) ) ) {
     return fail( ETIR_NO_DATA_PTR_PROVIDED, "contraction: null tensor pointer" );
@@ -1546,17 +1549,49 @@ int launch_contraction( ContractionPlan const & plan,
   if( plan.needs_aux && out_aux == nullptr ) {
     return fail( ETIR_NO_DATA_PTR_PROVIDED, "contraction: touch kernel needs the auxiliary tensor" );
   }
-  if( plan.packed ) {
+  if( !plan.order ) return enqueue( plan, left, right, out_aux, out, stream );
+  if( stream != nullptr ) {
     // under stream capture the operands are read in place: replays of a graph
-    // are ordered with nothing that uses the workspace outside it
+    // are ordered with nothing that uses the copies outside it
     hipStreamCaptureStatus l_cap = hipStreamCaptureStatusNone;
-    if( hipStreamIsCapturing( stream, &l_cap ) == hipSuccess && l_cap == hipStreamCaptureStatusNone ) {
-      return launch_packed( *plan.packed, left, right, out_aux, out, stream );
+    hipError_t const l_he = hipStreamIsCapturing( stream, &l_cap );
+    if( l_he != hipSuccess ) (void) hipGetLastError();
+    if( l_he != hipSuccess || l_cap != hipStreamCaptureStatusNone ) {
+      return enqueue( plan, left, right, out_aux, out, stream );
     }
-    (void) hipGetLastError();
   }
+  auto go = [&]() {
+    return plan.packed ? enqueue_packed( *plan.packed, left, right, out_aux, out, stream )
+                       : enqueue( plan, left, right, out_aux, out, stream );
+  };
+  if( ordered ) return go();
+  ExecOrder & l_o = *plan.order;
+  std::lock_guard< std::mutex > l_guard( l_o.lock );
+  if( !l_o.events && stream != nullptr ) {
+    // the first execution outside the null stream: those before were on it
+    if( l_o.ran ) ETIR_HIP_CHECK( hipEventRecord( l_o.done, nullptr ) );
+    l_o.events = true;
+  }
+  // also where the stream handle is the last execution's, which costs nothing:
+  // a handle names another stream once the first has been destroyed (its work
+  // may still run) or, for the per-thread default stream, in another thread
+  if( l_o.events && l_o.ran ) ETIR_HIP_CHECK( hipStreamWaitEvent( stream, l_o.done, 0 ) );
+  int const l_err = go();
+  // also after an error: what was enqueued still uses the plan's memory
+  l_o.ran = true;
+  if( l_o.events ) ETIR_HIP_CHECK( hipEventRecord( l_o.done, stream ) );
+  return l_err;
+}
+
+// The kernels of one execution, operands read in place.
+static int enqueue( ContractionPlan const & plan,
+                    void const            * left,
+                    void const            * right,
+                    void const            * out_aux,
+                    void                  * out,
+                    hipStream_t             stream ) {
   if( plan.split > 1 ) {
-    int l_err = launch_contraction( *plan.partial, left, right, nullptr, plan.d_ws, stream );
+    int l_err = enqueue( *plan.partial, left, right, nullptr, plan.d_ws, stream );
     if( l_err != ETIR_SUCCESS ) return l_err;
     ContractArgs const & p = plan.partial->args;
     SplitReduceArgs r{};

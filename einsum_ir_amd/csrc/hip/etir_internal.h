@@ -309,6 +309,19 @@ struct ContractArgs {
 
 struct PackedContraction;
 
+// Turns of a plan's executions, where they share memory of the plan (split-K
+// workspace, packed operands).  The lock keeps the launches of one execution
+// together; `done` orders executions on different streams.  As long as all of
+// them are on the null stream they are in order by themselves and record
+// nothing (a record between two kernels costs 3 us of the stream's time).
+struct ExecOrder {
+  std::mutex lock;
+  hipEvent_t done   = nullptr;
+  bool       ran    = false;     // an execution has been enqueued
+  bool       events = false;     // executions wait for `done` and record it
+};
+
+
 struct ContractionPlan {
   int32_t dtype_in   = ETIR_FP32;
   int32_t dtype_comp = ETIR_FP32;
@@ -353,6 +366,8 @@ struct ContractionPlan {
   std::shared_ptr< ContractionPlan > partial;
   // operands copied K-contiguous into a workspace first (null: read in place)
   std::shared_ptr< PackedContraction > packed;
+  // turns of the executions (null: they share no memory of the plan)
+  std::shared_ptr< ExecOrder > order;
   // tables and workspace live in a caller's region (DevicePlacement), not in
   // memory the plan allocated and frees
   bool    placed = false;
@@ -360,17 +375,13 @@ struct ContractionPlan {
 
 // A contraction over K-contiguous copies of one or both operands (slots: 0
 // left, 1 right): two permutations into the plan's workspace, then `cont` on
-// them.  One workspace for all executions: each waits for `done`, which the
-// one before recorded.
+// them.
 struct PackedContraction {
   ContractionPlan cont;
   PermutePlan perm[2];
   bool        use[2] = { false, false };
   void *      ws     = nullptr;
   int64_t     offset[2] = { 0, 0 };     // bytes into ws
-  std::mutex  lock;
-  hipEvent_t  done   = nullptr;
-  bool        ran    = false;
 };
 
 // Where a plan's device memory comes from when it may not allocate: a
@@ -447,7 +458,8 @@ int  launch_contraction( ContractionPlan const & plan,
                          void const            * right,
                          void const            * out_aux,
                          void                  * out,
-                         hipStream_t             stream );
+                         hipStream_t             stream,
+                         bool                    ordered );
 
 }  // namespace etir
 

@@ -121,7 +121,7 @@ extern "C" int etir_hip_contraction_execute_noalloc( int64_t         num_loops,
                                   strides_out, dtype_left, dtype_right, dtype_comp, dtype_out,
                                   ktype_first_touch, ktype_main, ktype_last_touch, l_plan, &l_place );
   if( l_err == ETIR_SUCCESS ) {
-    l_err = etir::launch_contraction( l_plan, left, right, out_aux, out, l_place.stream );
+    l_err = etir::launch_contraction( l_plan, left, right, out_aux, out, l_place.stream, false );
   }
   etir::release_contraction( l_plan );   // placed: frees nothing
   return l_err;

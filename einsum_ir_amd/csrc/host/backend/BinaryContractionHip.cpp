@@ -111,8 +111,8 @@ einsum_ir::err_t einsum_ir::backend::BinaryContractionHip::contract_async( void 
   if( !m_compiled ) {
     return err_t::CALLED_BEFORE_COMPILATION;
   }
-  int l_rc = etir_hip_contraction_execute( m_plan, i_tensor_left, i_tensor_right,
-                                           i_tensor_out_aux, io_tensor_out, m_stream );
+  auto l_execute = m_ordered ? etir_hip_contraction_execute_ordered : etir_hip_contraction_execute;
+  int l_rc = l_execute( m_plan, i_tensor_left, i_tensor_right, i_tensor_out_aux, io_tensor_out, m_stream );
   return static_cast< err_t >( l_rc );
 }
 

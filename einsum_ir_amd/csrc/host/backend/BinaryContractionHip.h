@@ -34,6 +34,9 @@ class einsum_ir::backend::BinaryContractionHip : public BinaryContraction {
 
     err_t compile();
 
+    //! the owner orders all executions (a tree's nodes)
+    bool m_ordered = false;
+
     /** Selects the HIP stream (hipStream_t as void*, nullptr = null stream). **/
     void set_stream( void * i_stream ) { m_stream = i_stream; }
 

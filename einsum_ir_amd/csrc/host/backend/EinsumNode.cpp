@@ -380,6 +380,8 @@ einsum_ir::err_t einsum_ir::backend::EinsumNode::compile_recursive() {
                   m_num_threads );
     static_cast< BinaryContractionHip * >( m_cont )->set_stream( m_stream );
     static_cast< BinaryContractionHip * >( m_cont )->m_cpx_dim_id = m_cpx_dim_id;
+    // evaluations of a tree share its intermediates and follow one another
+    static_cast< BinaryContractionHip * >( m_cont )->m_ordered = true;
     l_err = m_cont->compile();
     if( l_err != err_t::SUCCESS ) return l_err;
   }

@@ -16,7 +16,11 @@
  *     (reference src/constants.h:33-46).  A human-readable reason for the last
  *     failure on the calling thread is returned by etir_hip_last_error().
  *   - Plans are immutable after creation; executing one plan concurrently on
- *     different streams is safe.  Execution never allocates memory.
+ *     different streams or from several host threads is safe.  Executions of
+ *     a plan that computes in memory of its own (split K, copied operands)
+ *     take turns, ordered by an event; all others overlap.  A captured
+ *     execution is not ordered in this way: order the replays of its graph
+ *     with every other use of such a plan.  Execution never allocates memory.
  */
 #ifndef EINSUM_IR_HIP_H
 #define EINSUM_IR_HIP_H
@@ -101,8 +105,7 @@ typedef struct etir_plan_s * etir_plan_t;
  * The plan owns small device-resident offset tables (allocated here, never
  * during execution).  Where operands that the kernels would gather element by
  * element are large enough, it also owns K-contiguous copies of one or both
- * (at most 2 GiB), which every execution refills; executions of one plan on
- * different streams then take turns (ordered by an event).
+ * (at most 2 GiB), which every execution refills.
  */
 int etir_hip_contraction_create( int64_t         num_loops,
                                  int32_t const * dim_types,
@@ -133,6 +136,18 @@ int etir_hip_contraction_execute( etir_plan_t  plan,
                                   void const * out_aux,
                                   void       * out,
                                   void       * stream );
+
+/*
+ * The same for a caller that orders all executions of the plan itself, as a
+ * tree does with its nodes (no counterpart in the reference): no turns are
+ * taken, no event is recorded.
+ */
+int etir_hip_contraction_execute_ordered( etir_plan_t  plan,
+                                          void const * left,
+                                          void const * right,
+                                          void const * out_aux,
+                                          void       * out,
+                                          void       * stream );
 
 /*
  * Plans and executes one contraction without allocating device memory: the

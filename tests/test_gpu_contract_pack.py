@@ -7,6 +7,7 @@ Checker: torch.einsum in 64 bits on the same values.  Bars: fp32 1e-5 and
 bf16 2e-3 relative Frobenius (fp32 sums of exact products), fp64 1e-12.
 """
 import ctypes
+import threading
 
 import pytest
 
@@ -157,6 +158,35 @@ def test_packed_padding_is_cleared_before_the_first_execution(torch_cuda):
     eir.check(lib.etir_hip_stream_destroy(stream))
     for out in outs:
         assert _error(ref, out) <= TOL_FP32
+
+
+@pytest.mark.parametrize("own_streams", [False, True])
+def test_packed_from_several_threads(torch_cuda, own_streams):
+    """Three host threads on one plan, on the null stream or on streams of
+    their own: the copies and the kernel of an execution stay together."""
+    torch = torch_cuda
+    expr, sizes = "mk,nk->mn", dict(m=1023, n=1021, k=1019)
+    plan = _plan(expr, sizes, "float32")
+    assert "packed" in plan.describe(), plan.describe()
+    sets = [[_operands(torch, expr, sizes, "float32", 60 + 10 * t + i) for i in range(3)] for t in range(3)]
+    outs = [[torch.full(s[2], float("nan"), device="cuda") for s in x] for x in sets]
+    streams = [torch.cuda.Stream() if own_streams else None for _ in range(3)]
+    torch.cuda.synchronize()
+
+    def work(t):
+        for (a, b, _), out in zip(sets[t], outs[t]):
+            plan.execute(a, b, out, stream=streams[t])
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for x, y in zip(sets, outs):
+        for (a, b, _), out in zip(x, y):
+            assert _error(torch.einsum(expr, a.double(), b.double()), out) <= TOL_FP32
+    plan.close()
 
 
 def test_packed_on_a_recycled_stream(torch_cuda):

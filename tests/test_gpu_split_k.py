@@ -3,6 +3,8 @@ planner run the contraction as a partial contraction (outer K loops turned
 into batch loops writing workspace slices) plus a reduction that applies the
 touch kernels.  Checker: the CPU oracle (fp64 accumulation); fp32 relative
 Frobenius <= 1e-5, bf16 inputs <= 2e-3."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -143,3 +145,83 @@ def test_split_of_merged_k_loops_keeps_vector_loads(torch_cuda, oracle):
     of 61, which is one of 4 only where its inner part is."""
     _, desc = run_case(torch_cuda, oracle, "mkl,nkl->mn", dict(m=300, n=200, k=92, l=61), seed=78)
     assert "scalar" not in desc, desc
+
+
+def _mk_nk(torch, seed, m=256, n=192, k=32768):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    a, b = (torch.rand((r, k), device="cuda", generator=g) * 2 - 1 for r in (m, n))
+    return a, b, torch.full((m, n), float("nan"), device="cuda")
+
+
+def _split_plan(m=256, n=192, k=32768):
+    lp = eir.binary_loops("mk,nk->mn", dict(m=m, n=n, k=k))
+    plan = eir.ContractionPlan(lp["dim_types"], lp["sizes"], lp["strides_left"], lp["strides_right"],
+                               lp["strides_out"])
+    assert _split_of(plan.describe()) > 1 and "packed" not in plan.describe(), plan.describe()
+    return plan
+
+
+def _check_all(torch, sets):
+    torch.cuda.synchronize()
+    for a, b, out in sets:
+        ref = a.double() @ b.double().t().contiguous()
+        assert float((out.double() - ref).norm() / ref.norm()) <= 1e-5
+
+
+@pytest.mark.parametrize("null_first", [False, True])
+def test_split_on_several_streams(torch_cuda, null_first):
+    """One plan, other inputs on each of three streams in turn (the null stream
+    before them, or not), nothing waited for in between: each execution has the
+    workspace to itself."""
+    torch = torch_cuda
+    plan = _split_plan()
+    sets = [_mk_nk(torch, 80 + i) for i in range(9)]
+    streams = ([torch.cuda.default_stream()] * 2 if null_first else []) + [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+    for i, (a, b, out) in enumerate(sets):
+        plan.execute(a, b, out, stream=streams[i % len(streams)])
+    _check_all(torch, sets)
+    plan.close()
+
+
+@pytest.mark.parametrize("own_streams", [False, True])
+def test_split_from_several_threads(torch_cuda, own_streams):
+    """Three host threads on one plan, on the null stream or on streams of
+    their own: the two kernels of an execution stay together."""
+    torch = torch_cuda
+    plan = _split_plan()
+    sets = [[_mk_nk(torch, 100 + 10 * t + i) for i in range(4)] for t in range(3)]
+    streams = [torch.cuda.Stream() if own_streams else None for _ in range(3)]
+    torch.cuda.synchronize()
+
+    def work(t):
+        for a, b, out in sets[t]:
+            plan.execute(a, b, out, stream=streams[t])
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    _check_all(torch, [s for x in sets for s in x])
+    plan.close()
+
+
+def test_split_tree_nodes_on_a_stream(torch_cuda):
+    """Split nodes of a tree, evaluated repeatedly on a stream of the caller's:
+    the tree orders them."""
+    torch = torch_cuda
+    from einsum_ir_amd import host
+    sizes = dict(m=96, k=8192, n=64, l=4096, o=32)
+    g = torch.Generator(device="cuda").manual_seed(140)
+    a, b, c = (torch.randn(s, device="cuda", generator=g) for s in ((96, 8192), (8192, 4096), (64, 4096)))
+    out = torch.full((96, 64), float("nan"), device="cuda")
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    e = host.Expression("mk,kl,nl->mn", sizes, [(0, 1), (0, 1)], [a, b, c, out], dtype=eir.FP32, stream=stream)
+    for _ in range(3):
+        e.eval_async()
+    torch.cuda.synchronize()
+    e.close()
+    ref = a.double() @ b.double() @ c.double().t().contiguous()
+    assert float((out.double() - ref).norm() / ref.norm()) <= 1e-5

@@ -265,12 +265,13 @@ void perm_transpose16_kernel( PermArgs a ) {
 // consecutive elements per thread loaded one by one, fp32 4095 x 4095 ran at
 // 2.7 TB/s against 4.3 at 4096: 50.5 -> 37 us; bf16 31.4 -> 15 us).  All loads of a
 // thread are issued before the first LDS store.
-// NT: streaming stores, where the output rows are whole 128-byte lines (fp32
-// abcd->dbca 64^4 over tensors not in the caches 31.1 -> 21.7 us, 4096 x 4096
-// 31.3 -> 24.6 us); lines written in two pieces are slower that way (abcd->bdac
-// 36,48,36,512: 53.9 -> 77.8 us).  A compile-time choice: behind a run-time one
-// the compiler merges both stores into a plain one.
-template< typename T, int TI, int TO, bool VEC, bool NT >
+// Plain stores: streaming ones leave the caches to the input, but what reads the
+// output next loses more than that saves (fp32 abcd->dbca 64^4, other tensors on
+// every pass: 30.3 -> 28.4 us alone, with a permutation of its output after it
+// 51.0 -> 56.6, an elementwise pass 49.0 -> 55.8; 96,64,64,128 with a contraction
+// after it 206.6 -> 217.2), and lines written in two pieces are slower by
+// themselves (abcd->bdac 36,48,36,512: 53.9 -> 77.8 us).
+template< typename T, int TI, int TO, bool VEC >
 __global__ __launch_bounds__( kThreads )
 void perm_transpose_kernel( PermArgs a ) {
   static_assert( TI * TO == 4 * 4 * kThreads, "16 elements per thread" );
@@ -344,8 +345,7 @@ void perm_transpose_kernel( PermArgs a ) {
 #pragma unroll
           for( int l_e = 0; l_e < 4; l_e++ ) l_x.v[l_e] = Elem< T >::add( l_old.v[l_e], l_x.v[l_e] );
         }
-        if constexpr( NT ) store_stream( l_ptr, l_x );
-        else               *l_ptr = l_x;
+        *l_ptr = l_x;
       }
     }
   }
@@ -882,8 +882,12 @@ void perm_rows_kernel( PermArgs a ) {
 // 16-byte vector for bf16 and fp32, 32 bytes for fp64).  I is the type of
 // the element index the coordinates are decoded from: uint32_t when the
 // element count fits it (32-bit division), else uint64_t.
-// NT: streaming stores (COPY_VEC, fp32 and bf16, of whole 128-byte lines: abc->bac
-// 64,512,1024 bf16 27.1 -> 20.8 us; 512,512,96 fp32 41.0 -> 36.5 us).
+// NT: streaming stores (COPY_VEC, fp32 and bf16, of whole 128-byte lines), for
+// outputs of 128 MB and more, which the 256 MB Infinity Cache would not keep
+// beside the input for their reader: bf16 abc->bac, alone and with a contraction
+// of its output, plain -> streaming: 256,1024,1024 190.8 -> 185.9 and 329 -> 311
+// us; 128,512,1024 51.8 -> 49.0 and 85.2 -> 81.9; but 64,512,1024 27.7 -> 26.7 and
+// 44.6 -> 49.9.
 template< typename T, int VW, bool FILL, typename I, bool NT >
 __global__ __launch_bounds__( kThreads )
 void perm_gather_kernel( PermArgs a ) {
@@ -1063,15 +1067,14 @@ int launch_typed( PermutePlan const & p,
       }
     }
     else {
-      auto go = [&]( auto vec_c, auto nt_c ) {
-        constexpr bool VEC = decltype( vec_c )::value, NT = decltype( nt_c )::value;
-        if(      p.tr_shape == 1 ) hipLaunchKernelGGL( ( perm_transpose_kernel< T, 128, 32, VEC, NT > ), l_g, dim3( kThreads ), 0, stream, a );
-        else if( p.tr_shape == 2 ) hipLaunchKernelGGL( ( perm_transpose_kernel< T, 32, 128, VEC, NT > ), l_g, dim3( kThreads ), 0, stream, a );
-        else                       hipLaunchKernelGGL( ( perm_transpose_kernel< T, 64, 64, VEC, NT > ), l_g, dim3( kThreads ), 0, stream, a );
+      auto go = [&]( auto vec_c ) {
+        constexpr bool VEC = decltype( vec_c )::value;
+        if(      p.tr_shape == 1 ) hipLaunchKernelGGL( ( perm_transpose_kernel< T, 128, 32, VEC > ), l_g, dim3( kThreads ), 0, stream, a );
+        else if( p.tr_shape == 2 ) hipLaunchKernelGGL( ( perm_transpose_kernel< T, 32, 128, VEC > ), l_g, dim3( kThreads ), 0, stream, a );
+        else                       hipLaunchKernelGGL( ( perm_transpose_kernel< T, 64, 64, VEC > ), l_g, dim3( kThreads ), 0, stream, a );
       };
-      if( !a.vec_ok )         go( std::false_type(), std::false_type() );
-      else if( p.tr_lines && sizeof( T ) == 4 ) go( std::true_type(), std::true_type() );
-      else                    go( std::true_type(), std::false_type() );
+      if( a.vec_ok ) go( std::true_type() );
+      else           go( std::false_type() );
     }
   }
   else {
@@ -1086,7 +1089,7 @@ int launch_typed( PermutePlan const & p,
       constexpr bool l_fill = decltype( i_fill )::value;
       typedef typename decltype( i_idx )::type I;
       constexpr int l_wide = sizeof( T ) == 2 ? 8 : 4;
-      if( !l_fill && l_vw == l_wide && p.tr_lines && sizeof( T ) <= 4 ) {
+      if( !l_fill && l_vw == l_wide && p.nt_store && sizeof( T ) <= 4 ) {
         hipLaunchKernelGGL( ( perm_gather_kernel< T, l_wide, l_fill, I, true > ), l_g, dim3( kThreads ), 0, stream, a );
       }
       else if( l_vw == 8 ) hipLaunchKernelGGL( ( perm_gather_kernel< T, 8, l_fill, I, false > ), l_g, dim3( kThreads ), 0, stream, a );
@@ -1957,7 +1960,6 @@ int plan_permute( int64_t         num_dims,
     a.vec_ok = (    a.size_i % 4 == 0 && a.size_o % 4 == 0
                  && a.s_in_o % 4 == 0 && a.s_out_i % 4 == 0
                  && all_div4( l_dim_i, l_dim_o ) ) ? 1 : 0;
-    plan.tr_lines = whole_lines( l_dim_o );
     a.xcd_group = (    ( a.size_i * plan.elem_bytes ) % 128 != 0 || ( a.size_o * plan.elem_bytes ) % 128 != 0 )
                && a.tiles_i * a.tiles_o * a.num_batch_total >= 2048;
     return ETIR_SUCCESS;
@@ -1975,7 +1977,7 @@ int plan_permute( int64_t         num_dims,
     plan.mode = PermMode::COPY_VEC;
     a.vec_ok = 1;
     a.vec_wide = ( plan.elem_bytes == 2 && plan.size[l_n-1] % 8 == 0 && all_div( 8, l_n - 1, l_n - 1 ) ) ? 1 : 0;
-    plan.tr_lines = whole_lines( l_n - 1 );
+    plan.nt_store = whole_lines( l_n - 1 ) && plan.num_elements * plan.elem_bytes >= ( int64_t( 128 ) << 20 );
   }
   else {
     plan.mode = PermMode::GATHER;

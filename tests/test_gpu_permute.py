@@ -514,3 +514,26 @@ def test_pairs(torch_cuda, oracle, expr, sizes, dtype):
 def test_odd_transposes(torch_cuda, oracle, expr, sizes, dtype):
     for ktype in ([eir.COPY] if dtype == eir.BF16 else [eir.COPY, eir.ADD]):
         _check(torch_cuda, oracle, expr, sizes, dtype=dtype, ktype=ktype)
+
+
+@pytest.mark.parametrize("dtype", [eir.FP32, eir.BF16])
+@pytest.mark.parametrize("ktype", [eir.COPY, eir.ADD])
+@pytest.mark.parametrize("rows", [1023, 1024])
+def test_copies_from_128_mb_on(torch_cuda, dtype, ktype, rows):
+    """abc->bac with rows of whole 128-byte lines, just below 128 MB and at it,
+    from where the output is streamed past the caches; checked against torch."""
+    torch = torch_cuda
+    c = (128 << 20) // 1024 // 64 // eir.DTYPE_BYTES[dtype]
+    u = eir.unary_dims("abc->bac", dict(a=64, b=rows, c=c))
+    plan = eir.PermutePlan(u["sizes"], u["strides_in"], u["strides_out"], dtype=dtype, ktype=ktype)
+    assert "copy_vec" in plan.describe(), plan.describe()
+    # small whole numbers: sums are exact in both types
+    g = torch.Generator(device="cuda").manual_seed(3)
+    td = torch.float32 if dtype == eir.FP32 else torch.bfloat16
+    x, y = (torch.randint(-60, 60, s, device="cuda", generator=g).to(td) for s in ((64, rows, c), (rows, 64, c)))
+    ref = x.permute(1, 0, 2) + (y if ktype == eir.ADD else 0)
+    for _ in range(2):
+        out = y.clone()
+        plan.execute(x, out, stream=torch.cuda.current_stream())
+        assert torch.equal(out, ref)
+    plan.close()

@@ -466,9 +466,8 @@ int plan_contraction_impl( int64_t            num_loops,
     else if( n_tiles( TILE_BF16_128x128 ) >= l_cus ) plan.tile = TILE_BF16_128x128;
     else                                             plan.tile = TILE_BF16_64x64;
   }
-  // direct-to-LDS kernel: 16-byte vector modes on both operands, affine K,
-  // every byte offset below the buffer range (2^31), and enough 256 x 256
-  // tiles to give each CU at least one
+  // bf16 direct-to-LDS kernels: 16-byte vector modes on both operands, affine
+  // K, every byte offset below the buffer range (2^31)
   auto max_of = []( std::vector< int64_t > const & t ) {
     int64_t l_m = 0;
     for( int64_t l_v : t ) l_m = std::max( l_m, l_v );
@@ -493,11 +492,16 @@ int plan_contraction_impl( int64_t            num_loops,
   }
   // 256 x 256 tiles where their persistent scheduled loop runs (both operands
   // row-contiguous, whole tiles, plain fp32 output in 32-column runs: 4096 a
-  // side 109 us); everything else with a 128 x 128 tile per CU takes those,
-  // two workgroups per CU, against the generic 256 x 256 loop (one) and the
-  // register-staged tiles: mk,nk->mn 4096 a side 168 -> 126 us, 8192 x 1024 x
-  // 4096 82 -> 66 us, 4072 x 2048 x 2048 44 -> 38 us, 2304 x 2304 x 1024 20 ->
-  // 18 us; bf16 results (16-byte stores) 55 -> 36 us at 4072 x 2048 x 2048
+  // side 109 us) and, with row-contiguous operands, where its one-tile form
+  // walks a long K and leaves no large part of the last round of CUs idle
+  // (km,kn->mn, 256 against 128 tiles: 4072 x 4072 x 8192 230 / 314 us, 8184 x
+  // 4088 x 8192 463 / 595, x 4096 279 / 315; but 4072 x 4072 x 4096 142 / 144, x
+  // 2048 100 / 84, and 2552 x 8184 x 8192, 320 tiles, 422 / 411).  Everything
+  // else with a 128 x 128 tile per CU takes those, two workgroups per CU,
+  // against the generic 256 x 256 loop (one) and the register-staged tiles:
+  // mk,nk->mn 4096 a side 168 -> 126 us, 8192 x 1024 x 4096 82 -> 66 us, 4072 x
+  // 2048 x 2048 44 -> 38 us, 2304 x 2304 x 1024 20 -> 18 us; bf16 results
+  // (16-byte stores) 55 -> 36 us at 4072 x 2048 x 2048
   std::size_t l_run_n = 1;
   while( l_run_n < l_tn_out.size() && l_tn_out[l_run_n] == l_tn_out[l_run_n - 1] + 1 ) l_run_n++;
   bool const l_persistent =
@@ -508,7 +512,12 @@ int plan_contraction_impl( int64_t            num_loops,
       && 4 * ( max_of( l_tm_out ) + max_of( l_tn_out ) ) + 4 < ( int64_t( 1 ) << 32 );
   plan.scattered = l_run_n < 32 && l_run_n < l_tn_out.size() && l_tm_out.size() > 1
                 && l_tm_out[1] != l_tm_out[0] + int64_t( l_run_n );
-  if( l_dma_ok && l_persistent && n_tiles( TILE_BF16_DMA_256x256 ) >= l_cus ) plan.tile = TILE_BF16_DMA_256x256;
+  int64_t const l_t256 = n_tiles( TILE_BF16_DMA_256x256 );
+  double const l_last = double( l_t256 ) / double( ( l_t256 + l_cus - 1 ) / l_cus * l_cus + ( l_t256 == 0 ) );
+  bool const l_long_k = plan.mode_a == LOAD_VEC_MN && plan.mode_b == LOAD_VEC_MN
+                     && (    ( l_size_k >= 8192 && l_last >= 0.75 )
+                          || ( l_size_k >= 4096 && l_last >= 0.95 && l_t256 >= 2 * l_cus ) );
+  if( l_dma_ok && ( l_persistent || l_long_k ) && l_t256 >= l_cus ) plan.tile = TILE_BF16_DMA_256x256;
   else if( l_dma_ok && n_tiles( TILE_BF16_DMA_128x128 ) >= l_cus ) plan.tile = TILE_BF16_DMA_128x128;
   // the fp32 direct-to-LDS kernel: where the planner chose the 128 x 128 fp32
   // tile, under the same conditions (4-byte elements; the loads of the step

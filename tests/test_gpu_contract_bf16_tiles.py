@@ -55,6 +55,21 @@ def test_dma_128x128(torch_cuda, expr, sizes, bf16_out):
     assert _error(ref, got) <= (2 ** -8 if bf16_out else 1e-5)
 
 
+@pytest.mark.parametrize("sizes,bf16_out,kw", [
+    (dict(m=4072, n=4088, k=8192), False, {}),     # one ragged tile per CU
+    (dict(m=4096, n=4064, k=8200), True, {}),      # a last k step of 8
+    (dict(m=4096, n=4096, k=8192), False, dict(ktype_last_touch=eir.RELU)),
+    (dict(m=8184, n=4096, k=4096), True, {}),      # two rounds from a K of 4096 on
+])
+def test_dma_256x256_long_k(torch_cuda, sizes, bf16_out, kw):
+    """Row-contiguous operands with a long K that the persistent loop does not take."""
+    torch = torch_cuda
+    ref, got, desc = _run(torch, "km,kn->mn", sizes, torch.bfloat16 if bf16_out else torch.float32, **kw)
+    assert "bf16_dma_256x256" in desc and "persistent" not in desc, desc
+    ref = torch.relu(ref) if kw else ref
+    assert _error(ref, got) <= (2 ** -8 if bf16_out else 1e-5)
+
+
 def test_bf16_stores_relu_and_unaligned(torch_cuda):
     """ReLU in the 16-byte stores, and an output one element off alignment
     (element stores)."""

@@ -676,13 +676,15 @@ int plan_contraction_impl( int64_t            num_loops,
   // 90 on split K).  Fewer than 128 only up to K = 512: 128 x 128 x 256 takes
   // 5.1 us against 8.4 on 64 x 64 tiles, whose four workgroups walk K step by
   // step (K = 96: 3.9 against 4.8; 512: 7.3 against 8.8 split); from 768 on
-  // split K has more workgroups (K = 1024: 11.7 against 9.1)
+  // split K has more workgroups (K = 1024: 11.7 against 9.1).  Up to K = 96
+  // only one round of one workgroup per CU (256 tiles, 512 x 512: 4.2 us
+  // against 5.1; 484 tiles, 704 x 704: 5.6 against 5.3; K = 112: 5.6 against 5.8)
   {
     int64_t const l_t32 = n_tiles( TILE_F32_KWAVE_32x32 );
     bool const l_kw_ok = l_f32 && plan.tile != TILE_GEMV && plan.tile != TILE_SKINNY && plan.tile != TILE_PANEL && plan.mode_a == LOAD_VEC_K && plan.mode_b == LOAD_VEC_K && l_k_affine
                       && l_sk_a == 1 && l_sk_b == 1 && l_size_k % 16 == 0 && l_size_k >= 96
                       && l_size_k <= 4096 && n_tiles( plan.tile ) < l_cus
-                      && ( l_t32 >= l_cus / 2 || l_size_k <= 512 ) && l_t32 <= 2 * l_cus
+                      && ( l_t32 >= l_cus / 2 || l_size_k <= 512 ) && l_t32 <= ( l_size_k < 112 ? 1 : 2 ) * l_cus
                       && std::getenv( "ETIR_NO_KWAVE" ) == nullptr;
     if( l_kw_ok ) {
       // 8 waves up to K = 512, 16 above (config 1, K = 512: 7.58-7.65 us with

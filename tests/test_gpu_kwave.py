@@ -50,3 +50,10 @@ def test_kwave_few_tiles(torch_cuda, oracle, m, n, k):
     """Few tiles and a K of 96 to 512: waves whose K range is short or empty."""
     _, desc = run_case(torch_cuda, oracle, "mk,nk->mn", dict(m=m, n=n, k=k), seed=k)
     assert m == 1 or "f32_kwave_32x32" in desc, desc
+
+
+@pytest.mark.parametrize("n,k,taken", [(512, 96, True), (544, 96, False), (544, 112, True)])
+def test_kwave_short_k_takes_one_round(torch_cuda, oracle, n, k, taken):
+    """256 and 272 tiles: with a K of 96 no second workgroup per CU."""
+    _, desc = run_case(torch_cuda, oracle, "mk,nk->mn", dict(m=512, n=n, k=k), seed=k)
+    assert ("f32_kwave_32x32" in desc) == taken, desc

@@ -1233,7 +1233,8 @@ double plan_us( ContractionPlan const & plan, bool far, double flops, double byt
 // beside its bytes): aecf,bfde->abcd 24,24,12,12,12,12 fp32 12.5 -> 14.0 us,
 // eafd,fbec->abcd 42,42,21,21,21,21 fp32 46 -> 53 us.
 //
-// Never fails: without a gain, or without the memory, the plan stays as it is.
+// Never fails: without a gain, or where the copies would take more than an
+// eighth of the free device memory, the plan stays as it is.
 void try_pack( int64_t            num_loops,
                int32_t const    * dim_types,
                int64_t const    * sizes,
@@ -1442,7 +1443,11 @@ void try_pack( int64_t            num_loops,
     l_total += ( l_s * l_esz + 255 ) / 256 * 256;
   }
   Loops const & l_lp = l_best.loops;
-  if(    plan_contraction_impl( (int64_t) l_lp.type.size(), l_lp.type.data(), l_lp.size.data(), l_lp.s[0].data(),
+  std::size_t l_free = 0, l_device = 0;
+  if(    hipMemGetInfo( &l_free, &l_device ) != hipSuccess
+      // memory that a program is about to need stays free
+      || 8 * std::size_t( l_total ) > l_free
+      || plan_contraction_impl( (int64_t) l_lp.type.size(), l_lp.type.data(), l_lp.size.data(), l_lp.s[0].data(),
                                 l_lp.s[1].data(), l_lp.aux.data(), l_lp.out.data(), dtype_left, dtype_right,
                                 dtype_comp, dtype_out, ktype_first_touch, ktype_main, ktype_last_touch, allow_split,
                                 l_pk->cont, nullptr ) != ETIR_SUCCESS

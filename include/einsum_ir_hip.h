@@ -105,7 +105,8 @@ typedef struct etir_plan_s * etir_plan_t;
  * The plan owns small device-resident offset tables (allocated here, never
  * during execution).  Where operands that the kernels would gather element by
  * element are large enough, it also owns K-contiguous copies of one or both
- * (at most 2 GiB), which every execution refills.
+ * (at most 2 GiB and an eighth of the free device memory), which every
+ * execution refills.
  */
 int etir_hip_contraction_create( int64_t         num_loops,
                                  int32_t const * dim_types,

@@ -160,6 +160,32 @@ def test_packed_padding_is_cleared_before_the_first_execution(torch_cuda):
         assert _error(ref, out) <= TOL_FP32
 
 
+def test_copies_leave_memory_free(torch_cuda):
+    """With 512 MB of device memory left, 134 MB of copies are not taken."""
+    torch = torch_cuda
+    expr, sizes = "mk,nk->mn", dict(m=4095, n=4093, k=4091)
+    lib = eir.hip_lib()
+    _plan("mk,nk->mn", dict(m=16, n=16, k=16), "float32").close()
+    torch.cuda.empty_cache()
+    blocks = []
+    try:
+        while (take := torch.cuda.mem_get_info()[0] - (512 << 20)) >= 4 << 20:
+            block = ctypes.c_void_p()
+            eir.check(lib.etir_hip_malloc(ctypes.byref(block), min(take, 32 << 30)))
+            blocks.append(block)
+        full = _plan(expr, sizes, "float32")
+        left = torch.cuda.mem_get_info()[0]
+    finally:
+        for block in blocks:
+            eir.check(lib.etir_hip_free(block))
+    assert "packed" not in full.describe(), full.describe()
+    assert left >= 500 << 20, left
+    full.close()
+    plan = _plan(expr, sizes, "float32")
+    assert "packed" in plan.describe(), plan.describe()
+    plan.close()
+
+
 @pytest.mark.parametrize("own_streams", [False, True])
 def test_packed_from_several_threads(torch_cuda, own_streams):
     """Three host threads on one plan, on the null stream or on streams of

@@ -156,7 +156,7 @@ int etir_hip_plan_describe( etir_plan_t plan, char * buf, int64_t len ) {
       for( int l_k = 0; l_k < p.args.tile_nd; l_k++ ) {
         l_s += ( l_k ? "," : "" ) + std::to_string( p.args.tile_ext[l_k] );
       }
-      l_s += "] pad=" + std::to_string( p.args.tile_pad );
+      l_s += "] pad=" + std::to_string( p.args.tile_pad ) + " per=" + std::to_string( p.tile_per );
     }
     if( p.mode == etir::PermMode::TRANSPOSE && p.tr_shape != 0 ) {
       l_s += p.tr_shape == 1 ? " tile=128x32" : p.tr_shape == 2 ? " tile=32x128"

@@ -965,25 +965,24 @@ int launch_typed( PermutePlan const & p,
       return fail( ETIR_UNDEFINED_ERROR, "permute: grid too large" );
     }
     std::size_t const l_lds = std::size_t( a.tile_n + ( a.tile_n >> 6 ) * a.tile_pad ) * sizeof( T );
-    // batches of loads: 8 entries (4 of four elements); 2-byte elements on many
-    // workgroups one by one, whose other wavefronts hide the round trips
-    // already (abcde->eabcd 16,64,64,32,16 bf16: 49.3 us, 53.1 in batches; fp32
-    // equal; abcd->dcba 24,65,63,31 fp32 27.1 us one by one, 23.8 in batches of 8)
     auto go = [&]( auto v_c, auto per_c ) {
       hipLaunchKernelGGL( ( perm_tiled_kernel< T, decltype( v_c )::value, decltype( per_c )::value > ),
                           dim3( (uint32_t) l_blocks ), dim3( kThreads ), l_lds, stream, a );
     };
     std::integral_constant< int, 1 > const l_1{};
+    std::integral_constant< int, 2 > const l_2{};
     std::integral_constant< int, 4 > const l_4{};
     std::integral_constant< int, 8 > const l_8{};
-    bool const l_one = sizeof( T ) == 2 && l_blocks >= 512;
     if( p.tile_vw == 4 ) {
-      if( l_one ) go( l_4, l_1 );
-      else        go( l_4, l_4 );
+      if( p.tile_per == 1 )      go( l_4, l_1 );
+      else if( p.tile_per == 2 ) go( l_4, l_2 );
+      else                       go( l_4, l_4 );
     }
     else {
-      if( l_one ) go( l_1, l_1 );
-      else        go( l_1, l_8 );
+      if( p.tile_per == 1 )      go( l_1, l_1 );
+      else if( p.tile_per == 2 ) go( l_1, l_2 );
+      else if( p.tile_per == 4 ) go( l_1, l_4 );
+      else                       go( l_1, l_8 );
     }
   }
   else if( p.mode == PermMode::PAIR ) {
@@ -1308,15 +1307,19 @@ bool plan_tiled( PermutePlan & plan, int dim_i, int dim_o ) {
   };
   // small tensors in smaller tiles, about two per CU: with 4096-element tiles
   // a few CUs worked through four round trips to memory each while the
-  // others had nothing
-  int64_t const l_tile_max = std::max< int64_t >( 512, std::min< int64_t >( kPermTileMax, plan.num_elements / 512 ) );
+  // others had nothing (400 random tensors of 64 to 400,000 elements: geomean
+  // 0.76 of the time).  From 512 elements, but tiles of up to 1024 that hold
+  // whole runs stay whole: cut, their edges need the per-entry checks ([3,19,13]
+  // 3.8 -> 4.2 us as [3,10,13], 3.5 whole)
+  int64_t const l_tile_max  = std::max< int64_t >( 512, std::min< int64_t >( kPermTileMax, plan.num_elements / 512 ) );
+  int64_t const l_whole_max = std::max< int64_t >( 1024, l_tile_max );
   // tiles of kPermTileMax elements where the dims allow (grow the outermost
   // run dims): small tiles leave each workgroup too little work
   // first the run needs alone may exceed the limit: halve the largest extent,
   // the unit-stride dims' last (their multiples of 4 keep 16-byte accesses)
   int const l_ui = (int) ( std::find( l_td.begin(), l_td.end(), dim_i ) - l_td.begin() );
   int const l_uo = (int) ( std::find( l_td.begin(), l_td.end(), dim_o ) - l_td.begin() );
-  while( tile_n() > l_tile_max ) {
+  for( int64_t l_max = l_whole_max; tile_n() > l_max; l_max = l_tile_max ) {
     int l_big = -1;
     for( int l_k = 0; l_k < l_nt; l_k++ ) {
       if( l_k == l_ui || l_k == l_uo || l_e[l_k] <= 1 ) continue;
@@ -1325,6 +1328,9 @@ bool plan_tiled( PermutePlan & plan, int dim_i, int dim_o ) {
     if( l_big < 0 ) l_big = ( l_e[l_ui] >= l_e[l_uo] ) ? l_ui : l_uo;
     if( l_e[l_big] <= 1 ) return false;
     l_e[l_big] = ( l_e[l_big] + 1 ) / 2;
+    if( ( l_big == l_ui || l_big == l_uo ) && plan.size[l_td[l_big]] % 4 == 0 && l_e[l_big] > 4 ) {
+      l_e[l_big] = ( l_e[l_big] + 3 ) / 4 * 4;
+    }
   }
   // then grow the outermost run dims while the tile stays within the limit
   bool l_grew = true;
@@ -1333,7 +1339,8 @@ bool plan_tiled( PermutePlan & plan, int dim_i, int dim_o ) {
     for( int l_k = l_nt - 1; l_k >= 0; l_k-- ) {
       int64_t const l_cap = std::min< int64_t >( plan.size[l_td[l_k]], 128 );
       int64_t const l_new = std::min( l_cap, 2 * l_e[l_k] );
-      if( l_new > l_e[l_k] && tile_n() / l_e[l_k] * l_new <= l_tile_max ) {
+      int64_t const l_max = l_new == plan.size[l_td[l_k]] ? l_whole_max : l_tile_max;
+      if( l_new > l_e[l_k] && tile_n() / l_e[l_k] * l_new <= l_max ) {
         l_e[l_k] = l_new;
         l_grew = true;
       }
@@ -1493,6 +1500,17 @@ bool plan_tiled( PermutePlan & plan, int dim_i, int dim_o ) {
     if( l_d != dim_i && plan.s_in[l_d] % 4 != 0 ) a.vec_ok = 0;
     if( l_d != dim_o && plan.s_out[l_d] % 4 != 0 ) a.vec_ok = 0;
   }
+  // batches of loads: up to 8 entries (4 of four elements), no more than a
+  // thread has in the tile (loads of absent ones cost as much: bf16
+  // [3,13,6] -> [6,3,13], one entry a thread, 3.07 us in batches of 8, 2.54);
+  // 2-byte elements on many workgroups one by one, whose other wavefronts hide
+  // the round trips already (abcde->eabcd 16,64,64,32,16 bf16: 49.3 us, 53.1 in
+  // batches; fp32 equal; abcd->dcba 24,65,63,31 fp32 27.1 us one by one, 23.8 in
+  // batches of 8)
+  int64_t l_blocks = a.num_batch_total;
+  for( int l_k = 0; l_k < l_nt; l_k++ ) l_blocks *= a.tile_nblk[l_k];
+  int64_t const l_each = ( plan.elem_bytes == 2 && l_blocks >= 512 ) ? 1 : ( l_nv + kThreads - 1 ) / kThreads;
+  plan.tile_per = l_each <= 2 ? (int32_t) l_each : ( l_each <= 4 || l_vw == 4 ) ? 4 : 8;
   return true;
 }
 

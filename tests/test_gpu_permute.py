@@ -516,6 +516,20 @@ def test_odd_transposes(torch_cuda, oracle, expr, sizes, dtype):
         _check(torch_cuda, oracle, expr, sizes, dtype=dtype, ktype=ktype)
 
 
+@pytest.mark.parametrize("dtype,expr,sizes,tile", [
+    (eir.BF16, "abc->cab", dict(a=3, b=13, c=6), "[6,39] pad=0 per=1"),         # 234 elements: one entry a thread
+    (eir.BF16, "abcd->bdca", dict(a=13, b=3, c=19, d=3), "[3,19,13]"),          # 741 elements: a whole tile, not cut
+    (eir.FP32, "abcd->dbca", dict(a=3, b=18, c=6, d=2), "[2,108,3]"),           # grown to whole runs past 512
+    (eir.FP32, "abcd->bdac", dict(a=22, b=9, c=60, d=36), "[20,32,1]"),         # cut, in whole vectors
+    (eir.FP32, "abcd->dbca", dict(a=30, b=24, c=28, d=2), "per=2"),             # small tiles: 512 elements
+    (eir.FP64, "abcd->dcba", dict(a=33, b=40, c=40, d=31), "per=8"),            # large tensor: full batches
+])
+def test_small_tiles(torch_cuda, oracle, dtype, expr, sizes, tile):
+    for ktype in ([eir.COPY] if dtype == eir.BF16 else [eir.COPY, eir.ADD]):
+        desc = _check(torch_cuda, oracle, expr, sizes, dtype=dtype, ktype=ktype)
+        assert tile in desc, desc
+
+
 @pytest.mark.parametrize("dtype", [eir.FP32, eir.BF16])
 @pytest.mark.parametrize("ktype", [eir.COPY, eir.ADD])
 @pytest.mark.parametrize("rows", [1023, 1024])

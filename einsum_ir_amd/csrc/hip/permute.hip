@@ -271,7 +271,8 @@ void perm_transpose16_kernel( PermArgs a ) {
 // 51.0 -> 56.6, an elementwise pass 49.0 -> 55.8; 96,64,64,128 with a contraction
 // after it 206.6 -> 217.2), and lines written in two pieces are slower by
 // themselves (abcd->bdac 36,48,36,512: 53.9 -> 77.8 us).
-template< typename T, int TI, int TO, bool VEC >
+// ROWS (VEC): rows a thread loads at once, 1 or all 4.
+template< typename T, int TI, int TO, bool VEC, int ROWS >
 __global__ __launch_bounds__( kThreads )
 void perm_transpose_kernel( PermArgs a ) {
   static_assert( TI * TO == 4 * 4 * kThreads, "16 elements per thread" );
@@ -302,11 +303,8 @@ void perm_transpose_kernel( PermArgs a ) {
   if constexpr( VEC ) {
     int const l_c4 = l_t % RT;
     int const l_r  = l_t / RT;
-    // read: rows along o, 4 consecutive i per thread, fp32 all four rows at
-    // once; fp64 row by row (four 32-byte vectors at once 1-5 % slower), bf16
-    // too (8-byte vectors: 2540 x 1148 5.7 us, 6.6 at once; abc->acb
-    // 59,452,116 6.8 against 7.9)
-    constexpr int NB = sizeof( T ) == 4 ? 4 : 1;
+    // read: rows along o, 4 consecutive i per thread
+    constexpr int NB = ROWS;
 #pragma unroll
     for( int l_p0 = 0; l_p0 < 4; l_p0 += NB ) {
       Vec4< T > l_v[NB];
@@ -1068,14 +1066,20 @@ int launch_typed( PermutePlan const & p,
       }
     }
     else {
-      auto go = [&]( auto vec_c ) {
-        constexpr bool VEC = decltype( vec_c )::value;
-        if(      p.tr_shape == 1 ) hipLaunchKernelGGL( ( perm_transpose_kernel< T, 128, 32, VEC > ), l_g, dim3( kThreads ), 0, stream, a );
-        else if( p.tr_shape == 2 ) hipLaunchKernelGGL( ( perm_transpose_kernel< T, 32, 128, VEC > ), l_g, dim3( kThreads ), 0, stream, a );
-        else                       hipLaunchKernelGGL( ( perm_transpose_kernel< T, 64, 64, VEC > ), l_g, dim3( kThreads ), 0, stream, a );
+      auto go = [&]( auto vec_c, auto rows_c ) {
+        constexpr bool VEC  = decltype( vec_c )::value;
+        constexpr int  ROWS = decltype( rows_c )::value;
+        if(      p.tr_shape == 1 ) hipLaunchKernelGGL( ( perm_transpose_kernel< T, 128, 32, VEC, ROWS > ), l_g, dim3( kThreads ), 0, stream, a );
+        else if( p.tr_shape == 2 ) hipLaunchKernelGGL( ( perm_transpose_kernel< T, 32, 128, VEC, ROWS > ), l_g, dim3( kThreads ), 0, stream, a );
+        else                       hipLaunchKernelGGL( ( perm_transpose_kernel< T, 64, 64, VEC, ROWS > ), l_g, dim3( kThreads ), 0, stream, a );
       };
-      if( a.vec_ok ) go( std::true_type() );
-      else           go( std::false_type() );
+      std::integral_constant< int, 1 > const l_row{};
+      if( !a.vec_ok ) go( std::false_type(), l_row );
+      else if constexpr( sizeof( T ) == 4 ) {
+        if( p.tr_rows == 4 ) go( std::true_type(), std::integral_constant< int, 4 >() );
+        else                 go( std::true_type(), l_row );
+      }
+      else go( std::true_type(), l_row );
     }
   }
   else {
@@ -1982,6 +1986,15 @@ int plan_permute( int64_t         num_dims,
                  && all_div4( l_dim_i, l_dim_o ) ) ? 1 : 0;
     a.xcd_group = (    ( a.size_i * plan.elem_bytes ) % 128 != 0 || ( a.size_o * plan.elem_bytes ) % 128 != 0 )
                && a.tiles_i * a.tiles_o * a.num_batch_total >= 2048;
+    // fp32 loads all four rows of a thread at once, but not with 1152 to 2047
+    // workgroups, whose loads then queue (300 transposes of 10 to 80 MB, time
+    // at once / row by row: 480 x 30 x 352 11.7 / 10.1 us; 1200-1400 workgroups
+    // 1.06, 1400-1600 1.08, 1600-1800 1.04, up to 2047 1.0; below 512 0.9, above
+    // 2048 0.9-0.97).  fp64 row by row (four 32-byte vectors at once 1-5 %
+    // slower), bf16 too (8-byte vectors: 2540 x 1148 5.7 us, 6.6 at once;
+    // abc->acb 59,452,116 6.8 against 7.9)
+    int64_t const l_blocks = a.tiles_i * a.tiles_o * a.num_batch_total;
+    plan.tr_rows = ( plan.elem_bytes == 4 && ( l_blocks < 1152 || l_blocks >= 2048 ) ) ? 4 : 1;
     return ETIR_SUCCESS;
   }
 

@@ -516,6 +516,21 @@ def test_odd_transposes(torch_cuda, oracle, expr, sizes, dtype):
         _check(torch_cuda, oracle, expr, sizes, dtype=dtype, ktype=ktype)
 
 
+@pytest.mark.parametrize("expr,sizes,rows", [
+    ("abc->cba", dict(a=64, b=1151, c=64), 4),     # one 64 x 64 tile a workgroup
+    ("abc->cba", dict(a=64, b=1152, c=64), 1),
+    ("abc->cba", dict(a=64, b=2047, c=64), 1),
+    ("abc->cba", dict(a=64, b=2048, c=64), 4),
+    ("abc->cba", dict(a=32, b=1200, c=128), 1),    # 128 x 32
+    ("abc->cba", dict(a=128, b=1200, c=32), 1),    # 32 x 128
+])
+def test_transposed_rows_at_once(torch_cuda, oracle, expr, sizes, rows):
+    """fp32 vectors: the four rows of a thread loaded at once or one by one."""
+    for ktype in (eir.COPY, eir.ADD):
+        desc = _check(torch_cuda, oracle, expr, sizes, ktype=ktype)
+        assert "transpose" in desc and "batch=%d" % rows in desc, desc
+
+
 @pytest.mark.parametrize("dtype,expr,sizes,tile", [
     (eir.BF16, "abc->cab", dict(a=3, b=13, c=6), "[6,39] pad=0 per=1"),         # 234 elements: one entry a thread
     (eir.BF16, "abcd->bdca", dict(a=13, b=3, c=19, d=3), "[3,19,13]"),          # 741 elements: a whole tile, not cut

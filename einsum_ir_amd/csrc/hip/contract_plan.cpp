@@ -223,9 +223,10 @@ int plan_contraction_impl( int64_t            num_loops,
                            bool               allow_split,
                            ContractionPlan  & plan,
                            DevicePlacement  * place,
-                           bool               dry = false ) {
+                           bool               dry = false,
+                           bool               copied = false ) {
   // dry: tile, load modes and split (those of its partial contraction) only,
-  // no device memory
+  // no device memory; copied: operands of a packed contraction
   plan = ContractionPlan();
   plan.placed = ( place != nullptr );
 
@@ -484,10 +485,20 @@ int plan_contraction_impl( int64_t            num_loops,
   plan.tile_fallback = plan.tile;
   // fp64 direct-to-LDS kernel: both operands K-contiguous, byte offsets below
   // the buffer range (the loads of the step past the last one are issued
-  // too), and the 128 x 128 tiles fill the chip as well as the 64 x 64 ones
+  // too), and fewer rounds of tiles: a round of one 128 x 128 tile per CU takes
+  // as long as three of 64 x 64 ones (per unit of K 0.12 us, 0.04), also a last
+  // one that is nearly empty.  mk,nk->mn, 64 / 128 tiles: 2544 x 1539 x 2442 (4
+  // rounds, 2) 396 / 581 us, 3320 x 1491 x 574 (5, 2) 127 / 147, K = 98 with 9
+  // and 3 rounds 56 / 61; 252 tiles, K = 1534 (4, 1) 253 / 207.  Up to a K of 64
+  // loads and stores count, and the larger tiles only have to fill the chip (5
+  // rounds and 2, K = 54: 27.8 / 27.6; 6 and 2, K = 38: 27.8 / 24.2); so they do
+  // for copied operands (aecf,bfde->abcd 48,46,43,44,41,39, 272 tiles: 419 us
+  // packed on them, 862 in place)
+  auto rounds = [&]( int32_t t ) { return ( n_tiles( t ) + l_cus - 1 ) / l_cus; };
   if(    l_f64 && !l_cpx && plan.mode_a == LOAD_VEC_K && plan.mode_b == LOAD_VEC_K && l_k_affine && l_sk_a == 1
       && l_sk_b == 1 && 8 * ( std::max( max_of( l_tm_a ), max_of( l_tn_b ) ) + l_size_k + 64 ) < ( int64_t( 1 ) << 31 )
-      && score( TILE_F64_DMA_128x128 ) >= 0.9 * score( TILE_F64_64x64 ) ) {
+      && (    3 * rounds( TILE_F64_DMA_128x128 ) < rounds( TILE_F64_64x64 )
+           || ( ( copied || l_size_k <= 64 ) && score( TILE_F64_DMA_128x128 ) >= 0.9 * score( TILE_F64_64x64 ) ) ) ) {
     plan.tile = TILE_F64_DMA_128x128;
   }
   // 256 x 256 tiles where their persistent scheduled loop runs (both operands
@@ -850,7 +861,7 @@ int plan_contraction_impl( int64_t            num_loops,
         int l_err = plan_contraction_impl( (int64_t) l_pt.size(), l_pt.data(), l_psz.data(), l_pl.data(),
                                            l_pr.data(), l_pa.data(), l_po.data(), dtype_left, dtype_right,
                                            ETIR_FP32, ETIR_FP32, ETIR_KTYPE_ZERO, ETIR_KTYPE_MADD,
-                                           ETIR_KTYPE_UNDEFINED, false, *l_part, place, dry );
+                                           ETIR_KTYPE_UNDEFINED, false, *l_part, place, dry, copied );
         if( l_err != ETIR_SUCCESS ) {
           release_contraction( *l_part );
           return l_err;
@@ -1389,7 +1400,7 @@ void try_pack( int64_t            num_loops,
     if( plan_contraction_impl( (int64_t) l_lp.type.size(), l_lp.type.data(), l_lp.size.data(), l_lp.s[0].data(),
                                l_lp.s[1].data(), l_lp.aux.data(), l_lp.out.data(), dtype_left, dtype_right,
                                dtype_comp, dtype_out, ktype_first_touch, ktype_main, ktype_last_touch, allow_split,
-                               l_try, nullptr, true ) != ETIR_SUCCESS ) {
+                               l_try, nullptr, true, true ) != ETIR_SUCCESS ) {
       continue;
     }
     if( plan_rate( l_try, false ) == 0.0 || !in_vec( l_try.mode_a ) || !in_vec( l_try.mode_b ) ) continue;
@@ -1450,7 +1461,7 @@ void try_pack( int64_t            num_loops,
       || plan_contraction_impl( (int64_t) l_lp.type.size(), l_lp.type.data(), l_lp.size.data(), l_lp.s[0].data(),
                                 l_lp.s[1].data(), l_lp.aux.data(), l_lp.out.data(), dtype_left, dtype_right,
                                 dtype_comp, dtype_out, ktype_first_touch, ktype_main, ktype_last_touch, allow_split,
-                                l_pk->cont, nullptr ) != ETIR_SUCCESS
+                                l_pk->cont, nullptr, false, true ) != ETIR_SUCCESS
       || hipMalloc( &l_pk->ws, (std::size_t) l_total ) != hipSuccess
       // the padding's zeros are there when this returns: the fill runs on the
       // null stream, which a non-blocking stream's first execution does not

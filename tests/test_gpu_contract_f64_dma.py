@@ -55,6 +55,19 @@ def test_f64_dma(torch_cuda, expr, sizes):
     assert err <= TOL_FP64
 
 
+@pytest.mark.parametrize("m,n,k,taken", [
+    (2544, 1539, 66, False),     # 2 rounds of 128 x 128 tiles against 4 of 64 x 64
+    (2544, 1539, 64, True),
+    (2047, 2033, 66, True),      # 1 against 4
+    (3000, 2590, 98, True),      # 2 (504 tiles) against 8
+    (3000, 2689, 98, False),     # 3 (528) against 8
+])
+def test_f64_tile_rounds(torch_cuda, m, n, k, taken):
+    err, desc = _case(torch_cuda, "mk,nk->mn", dict(m=m, n=n, k=k))
+    assert ("f64_dma_128x128x16" in desc) == taken, desc
+    assert err <= TOL_FP64
+
+
 @pytest.mark.parametrize("first,last", [(eir.COPY, eir.UNDEFINED_KTYPE), (eir.ADD, eir.RELU),
                                         (eir.UNDEFINED_KTYPE, eir.ADD), (eir.ZERO, eir.RELU)])
 def test_f64_dma_touch_kernels(torch_cuda, first, last):

@@ -1,5 +1,8 @@
-// Instantiations of the direct-to-LDS bf16 contraction kernel: 256 x 256
-// tiles, 4 waves, one per (A load mode, B load mode) in {VEC_MN, VEC_K}.
+// Instantiations of the direct-to-LDS bf16 contraction kernel: 128 x 128 tiles
+// and 256 x 256 tiles, 4 waves, one per (A load mode, B load mode) in {VEC_MN,
+// VEC_K}.  The planner takes 256 x 256 tiles for VEC_MN x VEC_MN only; the
+// generic 64-wide loop on them and the 256 x 128 tiles run under the diagnostic
+// switches alone (ETIR_TILE, ETIR_DMA_VARIANT), 128 x 128 tiles being faster.
 #include "contract_dma.h"
 
 namespace etir {
@@ -57,7 +60,7 @@ int launch_contract_bf16_dma( int32_t ma, int32_t mb, int32_t variant, ContractA
                               uint32_t grid, hipStream_t stream ) {
   if( variant == 2 ) return launch_bf16_dma_256x128( ma, mb, a, grid, stream );
   if( variant == 4 ) return launch_bf16_dma_128x128( ma, mb, a, grid, stream );
-  if( variant == 3 && ma == LOAD_VEC_MN && mb == LOAD_VEC_MN && kern::persistent_dma_eligible( a, 256, 256 ) ) {
+  if( variant == 3 && ma == LOAD_VEC_MN && mb == LOAD_VEC_MN && persistent_dma_eligible( a, 256, 256 ) ) {
     static thread_local int s_dev = -1;
     static thread_local uint32_t s_cus = 256;
     int l_dev = 0;

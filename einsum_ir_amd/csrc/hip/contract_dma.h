@@ -865,11 +865,6 @@ void contract_dma_kernel( ContractArgs a ) {
 // compiler copy the accumulators into VGPRs); the others use
 // contract_dma_kernel.
 // ---------------------------------------------------------------------------
-__host__ __device__ inline bool persistent_dma_eligible( ContractArgs const & a, int BM, int BN ) {
-  return a.M % BM == 0 && a.N % BN == 0 && a.out_off32 && a.out_nt && !a.out_bf16
-      && a.first_touch == ETIR_KTYPE_ZERO && a.last_touch == ETIR_KTYPE_UNDEFINED;
-}
-
 template< int BM, int BN, int BK, int WM, int WN, int STAGES >
 __global__ __launch_bounds__( 64 * WM * WN, 1 )
 void contract_dma_persistent_kernel( ContractArgs a ) {

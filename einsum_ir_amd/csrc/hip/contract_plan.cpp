@@ -515,6 +515,7 @@ int plan_contraction_impl( int64_t            num_loops,
   // (16-byte stores) 55 -> 36 us at 4072 x 2048 x 2048
   std::size_t l_run_n = 1;
   while( l_run_n < l_tn_out.size() && l_tn_out[l_run_n] == l_tn_out[l_run_n - 1] + 1 ) l_run_n++;
+  // persistent_dma_eligible, before the kernel's arguments exist
   bool const l_persistent =
          plan.mode_a == LOAD_VEC_MN && plan.mode_b == LOAD_VEC_MN && dtype_out == ETIR_FP32
       && ktype_first_touch == ETIR_KTYPE_ZERO && ktype_last_touch == ETIR_KTYPE_UNDEFINED
@@ -563,7 +564,7 @@ int plan_contraction_impl( int64_t            num_loops,
     if( l_t_ok ) plan.tile = l_t;
   }
   // VEC_MN x VEC_MN runs the explicitly scheduled BK 32 / 4-stage main loop;
-  // the other pairings (VEC_K needs 64-wide k rows) the generic BK 64 / 2-stage one
+  // the other pairings (VEC_K needs 64-wide k rows; under ETIR_TILE) the generic BK 64 / 2-stage one
   // (3: the persistent variant of the scheduled loop, for contractions it
   // runs -- all tiles full, plain fp32 stores -- decided at launch)
   plan.dma_variant = ( plan.mode_a == LOAD_VEC_MN && plan.mode_b == LOAD_VEC_MN ) ? 3 : 0;
@@ -1139,9 +1140,7 @@ int plan_contraction_impl( int64_t            num_loops,
     // non-temporal output stores only where each store instruction of the
     // fast epilogue (32 consecutive columns per half-wave) writes whole
     // unit-stride runs: the output's columns are consecutive in groups of 32
-    std::size_t l_run = 1;
-    while( l_run < l_tn_out.size() && l_tn_out[l_run] == l_tn_out[l_run - 1] + 1 ) l_run++;
-    a.out_nt = ( l_run >= 32 && ( l_run % 32 == 0 || l_run == l_tn_out.size() ) ) ? 1 : 0;
+    a.out_nt = ( l_run_n >= 32 && ( l_run_n % 32 == 0 || l_run_n == l_tn_out.size() ) ) ? 1 : 0;
     if( char const * l_env = std::getenv( "ETIR_OUT_NT" ) ) a.out_nt = std::atoi( l_env ) != 0 ? 1 : 0;
   }
   // K of one step with plain output: the one-step form of the fp32
@@ -1173,9 +1172,7 @@ int plan_contraction_impl( int64_t            num_loops,
     a.out_bytes  = uint32_t( 4 * ( l_mo + l_no + 1 ) );
     a.panel_grid = int32_t( l_cus );
   }
-  if(    plan.tile == TILE_BF16_DMA_256x256 && plan.dma_variant == 3 && a.M % 256 == 0 && a.N % 256 == 0
-      && a.out_off32 && a.out_nt && !a.out_bf16 && a.first_touch == ETIR_KTYPE_ZERO
-      && a.last_touch == ETIR_KTYPE_UNDEFINED ) {
+  if( plan.tile == TILE_BF16_DMA_256x256 && plan.dma_variant == 3 && persistent_dma_eligible( a, 256, 256 ) ) {
     plan.desc += " persistent";
   }
   return ETIR_SUCCESS;

@@ -309,6 +309,13 @@ struct ContractArgs {
   int32_t  panel_grid;
 };
 
+// what the persistent bf16 direct-to-LDS kernel runs: whole tiles, plain fp32
+// output in unit-stride runs of 32 columns
+inline bool persistent_dma_eligible( ContractArgs const & a, int32_t bm, int32_t bn ) {
+  return a.M % bm == 0 && a.N % bn == 0 && a.out_off32 && a.out_nt && !a.out_bf16
+      && a.first_touch == ETIR_KTYPE_ZERO && a.last_touch == ETIR_KTYPE_UNDEFINED;
+}
+
 struct PackedContraction;
 
 // Turns of a plan's executions, where they share memory of the plan (split-K
@@ -322,7 +329,6 @@ struct ExecOrder {
   bool       ran    = false;     // an execution has been enqueued
   bool       events = false;     // executions wait for `done` and record it
 };
-
 
 struct ContractionPlan {
   int32_t dtype_in   = ETIR_FP32;

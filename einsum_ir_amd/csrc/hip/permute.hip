@@ -1672,7 +1672,10 @@ int plan_permute( int64_t         num_dims,
 
   // a dim p of size 2 innermost on one side, on the other side not, and a
   // dim u next to it that is unit-stride there: pairs (interleaved <-> planar
-  // complex tensors), runs of at least 64
+  // complex tensors), runs of at least 64, where the tiled kernel stops.  Also at
+  // 64, where 16 of a workgroup's 256 threads move the run (360 permutations,
+  // runs of 64 to 2000, 8 thousand to 16 million elements, all types, both
+  // directions: 0.54 of the tiled kernel's time in the geomean, 0.85 at most)
   for( int l_p = 0; l_p < l_n; l_p++ ) {
     if( plan.size[l_p] != 2 || ( plan.s_in[l_p] == 1 ) == ( plan.s_out[l_p] == 1 ) ) continue;
     bool const l_split = plan.s_in[l_p] == 1;

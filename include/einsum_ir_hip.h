@@ -106,7 +106,9 @@ typedef struct etir_plan_s * etir_plan_t;
  * during execution).  Where operands that the kernels would gather element by
  * element are large enough, it also owns K-contiguous copies of one or both
  * (at most 2 GiB and an eighth of the free device memory), which every
- * execution refills.
+ * execution refills; creating such a plan takes 0.2 to 1.1 ms (trial plans, two
+ * permutation plans, the memory) instead of 0.05 to 0.2.  A captured execution
+ * reads its operands in place.
  */
 int etir_hip_contraction_create( int64_t         num_loops,
                                  int32_t const * dim_types,

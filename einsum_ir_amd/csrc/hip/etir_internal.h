@@ -149,7 +149,6 @@ struct PermutePlan {
   int32_t  tr_shape = 0;                 // TRANSPOSE: tile 64 x 64 (0), 128 x 32 (1) or 32 x 128 (2), i x o;
                                          // 2-byte elements with 16-byte reads: 128 x 64 (3), 128 x 32 (4)
   int32_t  tr_rows = 1;                  // TRANSPOSE, tr_shape 0 to 2 with vectors: rows a thread loads at once (1 or 4)
-  bool     tr_stream = false;            // TRANSPOSE, tr_rows 4: streaming (non-temporal) input loads
   bool     nt_store = false;             // COPY_VEC: streaming (non-temporal) output stores
   int64_t  rows_len = 0;                 // ROWS: row length (elements of the shared unit-stride dim)
 };

@@ -99,14 +99,6 @@ __device__ inline void store_stream( V * p, V const & v ) {
   }
 }
 
-// 16-byte load of a line that is not read again
-template< typename V >
-__device__ inline V load_stream( V const * p ) {
-  static_assert( sizeof( V ) == 16, "one 16-byte vector" );
-  typedef uint32_t u32x4 __attribute__( ( ext_vector_type( 4 ) ) );
-  return __builtin_bit_cast( V, __builtin_nontemporal_load( reinterpret_cast< u32x4 const * >( p ) ) );
-}
-
 // Type of an element held between its load and its store: 2-byte elements
 // take a register each.  Packed in pairs, the second load into a register
 // waits for the first (bf16 4095 x 4095: 31 us packed, 15 us not).
@@ -279,10 +271,8 @@ void perm_transpose16_kernel( PermArgs a ) {
 // 51.0 -> 56.6, an elementwise pass 49.0 -> 55.8; 96,64,64,128 with a contraction
 // after it 206.6 -> 217.2), and lines written in two pieces are slower by
 // themselves (abcd->bdac 36,48,36,512: 53.9 -> 77.8 us).
-// STREAM (fp32 vectors): streaming input loads, which leave the caches to the
-// output; a compile-time choice.
 // ROWS (VEC): rows a thread loads at once, 1 or all 4.
-template< typename T, int TI, int TO, bool VEC, int ROWS, bool STREAM >
+template< typename T, int TI, int TO, bool VEC, int ROWS >
 __global__ __launch_bounds__( kThreads )
 void perm_transpose_kernel( PermArgs a ) {
   static_assert( TI * TO == 4 * 4 * kThreads, "16 elements per thread" );
@@ -323,9 +313,7 @@ void perm_transpose_kernel( PermArgs a ) {
         int64_t const l_o = l_o0 + l_r + ( kThreads / RT ) * ( l_p0 + l_p );
         int64_t const l_i = l_i0 + 4 * l_c4;
         if( l_o < a.size_o && l_i < a.size_i ) {
-          Vec4< T > const * l_p4 = reinterpret_cast< Vec4< T > const * >( l_in + l_o * a.s_in_o + l_i );
-          if constexpr( STREAM ) l_v[l_p] = load_stream( l_p4 );
-          else                   l_v[l_p] = *l_p4;
+          l_v[l_p] = *reinterpret_cast< Vec4< T > const * >( l_in + l_o * a.s_in_o + l_i );
         }
       }
 #pragma unroll
@@ -1078,25 +1066,20 @@ int launch_typed( PermutePlan const & p,
       }
     }
     else {
-      auto go = [&]( auto vec_c, auto rows_c, auto stream_c ) {
-        constexpr bool VEC    = decltype( vec_c )::value;
-        constexpr int  ROWS   = decltype( rows_c )::value;
-        constexpr bool STREAM = decltype( stream_c )::value;
-        if(      p.tr_shape == 1 ) hipLaunchKernelGGL( ( perm_transpose_kernel< T, 128, 32, VEC, ROWS, STREAM > ), l_g, dim3( kThreads ), 0, stream, a );
-        else if( p.tr_shape == 2 ) hipLaunchKernelGGL( ( perm_transpose_kernel< T, 32, 128, VEC, ROWS, STREAM > ), l_g, dim3( kThreads ), 0, stream, a );
-        else                       hipLaunchKernelGGL( ( perm_transpose_kernel< T, 64, 64, VEC, ROWS, STREAM > ), l_g, dim3( kThreads ), 0, stream, a );
+      auto go = [&]( auto vec_c, auto rows_c ) {
+        constexpr bool VEC  = decltype( vec_c )::value;
+        constexpr int  ROWS = decltype( rows_c )::value;
+        if(      p.tr_shape == 1 ) hipLaunchKernelGGL( ( perm_transpose_kernel< T, 128, 32, VEC, ROWS > ), l_g, dim3( kThreads ), 0, stream, a );
+        else if( p.tr_shape == 2 ) hipLaunchKernelGGL( ( perm_transpose_kernel< T, 32, 128, VEC, ROWS > ), l_g, dim3( kThreads ), 0, stream, a );
+        else                       hipLaunchKernelGGL( ( perm_transpose_kernel< T, 64, 64, VEC, ROWS > ), l_g, dim3( kThreads ), 0, stream, a );
       };
       std::integral_constant< int, 1 > const l_row{};
-      std::integral_constant< int, 4 > const l_rows{};
-      std::true_type  const l_yes{};
-      std::false_type const l_no{};
-      if( !a.vec_ok ) go( l_no, l_row, l_no );
+      if( !a.vec_ok ) go( std::false_type(), l_row );
       else if constexpr( sizeof( T ) == 4 ) {
-        if( p.tr_stream )         go( l_yes, l_rows, l_yes );
-        else if( p.tr_rows == 4 ) go( l_yes, l_rows, l_no );
-        else                      go( l_yes, l_row, l_no );
+        if( p.tr_rows == 4 ) go( std::true_type(), std::integral_constant< int, 4 >() );
+        else                 go( std::true_type(), l_row );
       }
-      else go( l_yes, l_row, l_no );
+      else go( std::true_type(), l_row );
     }
   }
   else {
@@ -1647,11 +1630,11 @@ int plan_permute( int64_t         num_dims,
     }
     return true;
   };
-  // rows along dim d of the tensor with strides st are whole 128-byte lines
-  auto whole_lines = [&]( int d, int64_t const * st ) {
+  // output rows along dim d are whole 128-byte lines
+  auto whole_lines = [&]( int d ) {
     bool l_ok = ( plan.size[d] * plan.elem_bytes ) % 128 == 0;
     for( int l_di = 0; l_di < l_n; l_di++ ) {
-      l_ok = l_ok && ( l_di == d || ( st[l_di] * plan.elem_bytes ) % 128 == 0 );
+      l_ok = l_ok && ( l_di == d || ( plan.s_out[l_di] * plan.elem_bytes ) % 128 == 0 );
     }
     return l_ok;
   };
@@ -2015,19 +1998,6 @@ int plan_permute( int64_t         num_dims,
     // abc->acb 59,452,116 6.8 against 7.9)
     int64_t const l_blocks = a.tiles_i * a.tiles_o * a.num_batch_total;
     plan.tr_rows = ( plan.elem_bytes == 4 && ( l_blocks < 1152 || l_blocks >= 2048 ) ) ? 4 : 1;
-    // fp32 tensors of 48 MB and more with whole lines on both sides, tr_rows 4,
-    // stream their input: from there on, input, output and what is read next do
-    // not all stay in the 256 MB Infinity Cache, and the output is what a reader
-    // finds there.  abcd->dbca 64^4, plain / streamed loads: alone 30.1 / 28.5 us
-    // (other tensors on every pass), 30.5 / 25.6 (three in turn), with a
-    // permutation after it 53.9 / 49.7, between two elementwise passes 76.1 /
-    // 70.2; 48 to 256 MB 0.8-1.0 of the time throughout but 80 to 88 MB between
-    // elementwise passes, 1.02-1.09.  At 40 MB an input read again is still cached
-    // (14.0 / 18.6); lines in two tiles are fetched twice (60,64,64,68 with a
-    // permutation after it 75.6 / 86.5)
-    plan.tr_stream = (    plan.elem_bytes == 4 && plan.tr_rows == 4 && a.vec_ok
-                       && plan.num_elements * plan.elem_bytes >= ( int64_t( 48 ) << 20 )
-                       && whole_lines( l_dim_i, plan.s_in ) && whole_lines( l_dim_o, plan.s_out ) );
     return ETIR_SUCCESS;
   }
 
@@ -2043,7 +2013,7 @@ int plan_permute( int64_t         num_dims,
     plan.mode = PermMode::COPY_VEC;
     a.vec_ok = 1;
     a.vec_wide = ( plan.elem_bytes == 2 && plan.size[l_n-1] % 8 == 0 && all_div( 8, l_n - 1, l_n - 1 ) ) ? 1 : 0;
-    plan.nt_store = whole_lines( l_n - 1, plan.s_out ) && plan.num_elements * plan.elem_bytes >= ( int64_t( 128 ) << 20 );
+    plan.nt_store = whole_lines( l_n - 1 ) && plan.num_elements * plan.elem_bytes >= ( int64_t( 128 ) << 20 );
   }
   else {
     plan.mode = PermMode::GATHER;

@@ -531,31 +531,6 @@ def test_transposed_rows_at_once(torch_cuda, oracle, expr, sizes, rows):
         assert "transpose" in desc and "batch=%d" % rows in desc, desc
 
 
-@pytest.mark.parametrize("ktype", [eir.COPY, eir.ADD])
-@pytest.mark.parametrize("a,b,c,d,stream", [
-    (64, 47, 64, 64, False), (64, 48, 64, 64, True),     # just below 48 MB, and at it
-    (32, 64, 64, 128, True), (128, 64, 64, 32, True),    # 128 x 32 and 32 x 128 tiles
-    (64, 64, 64, 60, False), (60, 64, 64, 64, False),    # rows that split lines, on one side
-    (96, 32, 36, 160, True),                             # ragged tiles
-])
-def test_transposes_that_stream_their_input(torch_cuda, a, b, c, d, stream, ktype):
-    torch = torch_cuda
-    u = eir.unary_dims("abcd->dbca", dict(a=a, b=b, c=c, d=d))
-    plan = eir.PermutePlan(u["sizes"], u["strides_in"], u["strides_out"], ktype=ktype)
-    assert "transpose" in plan.describe() and ("stream" in plan.describe()) == stream, plan.describe()
-    g = torch.Generator(device="cuda").manual_seed(5)
-    x = torch.randint(-1000, 1000, (a, b, c, d), device="cuda", generator=g).float()
-    y = torch.randint(-1000, 1000, (d, b, c, a), device="cuda", generator=g).float()
-    ref = x.permute(3, 1, 2, 0) + (y if ktype == eir.ADD else 0)
-    for _ in range(2):
-        x += 1                                           # new values in the same buffer
-        ref += 1
-        out = y.clone()
-        plan.execute(x, out, stream=torch.cuda.current_stream())
-        assert torch.equal(out, ref)
-    plan.close()
-
-
 @pytest.mark.parametrize("dtype,expr,sizes,tile", [
     (eir.BF16, "abc->cab", dict(a=3, b=13, c=6), "[6,39] pad=0 per=1"),         # 234 elements: one entry a thread
     (eir.BF16, "abcd->bdca", dict(a=13, b=3, c=19, d=3), "[3,19,13]"),          # 741 elements: a whole tile, not cut
